@@ -228,3 +228,49 @@ def test_streamed_reduction_tail(gpu, k):
     b = store[:, :, :k].transpose(1, 2)          # [batch, k, n], column stride `pitch`
     bd = store.to(gpu)[:, :, :k].transpose(1, 2)
     assert bits_equal(capi.bmm(a.to(gpu), bd), ob.sequential_bmm(a, b))
+
+
+def _operand(form, batch, rows, k, g, device):
+    """Logical [batch, rows, k] fp16 operand stored with steps adjacent, with rows
+    adjacent (both at odd pitches and offsets), or with neither."""
+    if form == "steps":
+        t = torch.randn(batch, rows, k + 3, generator=g).half()
+        return t[:, :, 1:1 + k], t.to(device)[:, :, 1:1 + k]
+    if form == "rows":
+        t = torch.randn(batch, k, rows + 5, generator=g).half()
+        return t[:, :, 3:3 + rows].transpose(1, 2), t.to(device)[:, :, 3:3 + rows].transpose(1, 2)
+    t = torch.randn(batch, rows, 2 * k, generator=g).half()
+    return t[:, :, ::2], t.to(device)[:, :, ::2]
+
+
+@pytest.mark.parametrize("batch,m,n", [(2, 33, 31), (1, 47, 100), (130, 66, 70), (1, 1472, 1470)])
+@pytest.mark.parametrize("k", [1, 31, 32, 34, 64, 67, 130, 259])
+@pytest.mark.parametrize("fa,fb", [("steps", "steps"), ("rows", "rows"), ("steps", "rows"), ("rows", "steps"),
+                                   ("neither", "rows"), ("steps", "neither")])
+def test_bmm_load_forms(gpu, batch, m, n, k, fa, fb):
+    """Every pair of operand load forms at both tile sizes (the last two shapes
+    give 512 or more 64 x 64 tiles), with partial row tiles, reductions around
+    the 32, 64 and 128-step chunks and remainders of 4 and 8 steps, operands at
+    2-byte alignment: the bits of the sequential sum."""
+    from thintnpu_amd import capi
+    if batch * m * n * k > 130 * 66 * 70 * 130:
+        pytest.skip("the same chunk counts run at the smaller shapes")
+    g = gen(batch * 7 + m + k)
+    a, ad = _operand(fa, batch, m, k, g, gpu)
+    b, bd = _operand(fb, batch, n, k, g, gpu)
+    got = capi.bmm(ad, bd.transpose(1, 2))
+    assert bits_equal(got, ob.sequential_bmm(a, b.transpose(1, 2)))
+
+
+@pytest.mark.parametrize("c0,key,tokens", [(8, 24, 70), (32, 64, 33), (24, 48, 40), (16, 48, 1100)])
+def test_blocked_widths(gpu, c0, key, tokens):
+    """q^T k over operands blocked by 8, 32 (loaded in runs) and 24 (gathered)
+    channels, and over enough tokens for several tiles a block."""
+    from thintnpu_amd import capi
+    source = torch.randn(2, 2 * key // c0, tokens, c0, generator=gen(c0 + key)).half()
+    q, k = source.to(gpu).split((key // c0, key // c0), 1)
+    qr, kr = source.split((key // c0, key // c0), 1)
+    assert bits_equal(capi.layout_bmm(q, k, True, False, False), ob.layout_bmm(qr, kr, True, False, False))
+    # a range of channels that starts inside a block
+    got = capi.layout_bmm(q, k, True, False, False, 0, 4, 20, 4, 20)
+    assert bits_equal(got, ob.layout_bmm(qr, kr, True, False, False, 0, 4, 20, 4, 20))

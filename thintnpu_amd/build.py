@@ -38,6 +38,9 @@ HIP_FLAGS = [
     # the kernels spell out (e.g. the unfused-chain intermediates) survives.
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # matrix accumulators in VGPRs: no copies between the register halves around
+    # short product loops
+    "-mllvm", "-amdgpu-mfma-vgpr-form",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
     f"-I{INCLUDE}", f"-I{HIP_SRC}",
 ]

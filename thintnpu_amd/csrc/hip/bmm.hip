@@ -6,14 +6,15 @@
 // fp32 sum of its k products taken in reduction order 0, 1, ..., K-1 from a
 // zero start, then one round-to-nearest-even cast to fp16.  fp16 x fp16
 // products are exact in fp32 (22 significant bits, exponents far from the fp32
-// limits), so fma(a, b, acc) rounds exactly like acc + a * b and the per-output
-// chain of fmas reproduces the sequential sum bit for bit.  This rules out
-// MFMA tiles (their internal summation order differs) and any split of the
-// reduction; the parallelism is across outputs only.  The attention shapes are
-// small (a [4, 64, 400] x [4, 400, 400] product is 41 M fmas), so a product
-// is bound by the latency of its K-long dependent fma chains (about 32 cycles
-// per dependent fp32 fma on gfx950) and by memory latency, not by VALU
-// throughput.
+// limits), so fma(a, b, acc) rounds exactly like acc + a * b and a per-output
+// chain of fmas reproduces the sequential sum bit for bit.  On gfx950
+// v_mfma_f32_16x16x4_f32 is such a chain: it adds its four products to the
+// accumulator one after the other in ascending k, one fp32 rounding each
+// (compared with fmaf chains over 204,800 outputs of 64-256 steps: normal,
+// wide-exponent, cancelling, signed-zero, subnormal and non-finite fp16
+// operands, no bit differs).  The fp16 matrix instructions are not, and a
+// split of the reduction is not either, so the operands are widened to fp32
+// and the parallelism is across outputs only.
 #include "common.h"
 
 #include <string.h>
@@ -41,392 +42,615 @@ struct Mat {
   int64_t batch;
   uint32_t row_origin, col_origin, row_group, col_group;
   Axis row, col;
-  __device__ __forceinline__ int64_t at(uint32_t b, uint32_t r, uint32_t c) const {
-    return (int64_t)b * batch + row.at(r + row_origin + b * row_group) + col.at(c + col_origin + b * col_group);
-  }
 };
 
-constexpr uint32_t kBmmThreads = 256;  // 4 waves; wave w owns rows [w * RM, w * RM + RM) of the tile
-constexpr uint32_t kBmmCols = 64;      // one output column per lane
-constexpr uint32_t kBmmDepth = 32;     // reduction steps staged per LDS round
+// ---------------------------------------------------------------- matrix-core product
+// One operand of the product as the kernels read it: `rows` logical rows, each
+// K steps long.
+struct Side {
+  const _Float16* p;
+  int64_t batch;
+  int64_t hop;  // bytes from a chunk of steps (bmm_kernel) or a tile of rows (bmm_short_kernel's P) to the next
+  uint32_t row_origin, step_origin, row_group, step_group, rows;
+  bool steps_near;  // the smaller stride is along the steps
+  Axis row, step;
+};
 
+// The output with the axis that is contiguous in memory as `p` (the matrix
+// instruction gives a lane 4 consecutive rows of its tile, so that axis rides
+// on the instruction's rows) and the other as `q`.
 struct BmmPlan {
-  Mat a, b, y;          // a: [batch, m, k], b: [batch, k, n], y: [batch, m, n]
-  uint32_t m, n, k;
-  uint32_t mtiles, ntiles;
-  bool a_kfast, b_kfast;  // stage along k (the operand's smaller stride is on k)
-  // streamed b: bytes from b.p to the end of its storage, vectors per
-  // contiguous run along k (0 = one run) and the byte jump after a run
-  uint32_t b_bytes, b_vrun, b_vjump;
-  FastDiv div_mt, div_nt;  // streamed form: block index -> (batch, row tile, column tile)
+  Side P, Q;
+  _Float16* y;
+  int64_t ybatch;
+  uint32_t yp_group;  // p indexes between batch entries (grouped blocked outputs)
+  uint32_t y_vec;     // runs of 4 * W outputs along p from multiples of 4 * W are contiguous
+  Axis yp, yq;
+  uint32_t k;
+  uint32_t span;      // bmm_short_kernel: P tiles per block,
+  int64_t yhop;       // and output elements from one to the next
+  uint32_t ptiles;
+  FastDiv pblocks, qtiles;
 };
 
-// Output tile of 4 * RM rows x 64 columns per block.  A and B are staged as
-// fp32 in LDS, kBmmDepth reduction steps at a time; each step is one LDS
-// column read per lane, RM broadcast reads and RM fmas.
-template <int RM>
-__global__ __launch_bounds__(kBmmThreads) void bmm_kernel(BmmPlan p) {
-  constexpr uint32_t TM = 4 * RM;
-  constexpr uint32_t kAPitch = TM + 4;  // wave w's RM floats stay 4*RM-byte aligned
-  constexpr uint32_t kBPitch = kBmmCols + 1;
-  __shared__ __attribute__((aligned(16))) float As[kBmmDepth][kAPitch];
-  __shared__ float Bs[kBmmDepth][kBPitch];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  uint32_t t = blockIdx.x;
-  const uint32_t nt = t % p.ntiles;
-  t /= p.ntiles;
-  const uint32_t mt = t % p.mtiles;
-  const uint32_t bt = t / p.mtiles;
-  const uint32_t i0 = mt * TM, j0 = nt * kBmmCols;
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
 
-  // B staging: each thread's columns are fixed for the whole block
-  int64_t bcol[kBmmDepth * kBmmCols / kBmmThreads];
-  constexpr uint32_t kBPer = kBmmDepth * kBmmCols / kBmmThreads;  // 8
-#pragma unroll
-  for (uint32_t s = 0; s < kBPer; ++s) {
-    const uint32_t e = tid + s * kBmmThreads;
-    const uint32_t jj = p.b_kfast ? e / kBmmDepth : e % kBmmCols;
-    const uint32_t j = min(j0 + jj, p.n - 1);
-    bcol[s] = (int64_t)bt * p.b.batch + p.b.col.at(j + p.b.col_origin + bt * p.b.col_group);
-  }
+constexpr uint32_t kBmmThreads = 256;  // 4 waves, 2 x 2 over the block's tile
 
-  float acc[RM];
-#pragma unroll
-  for (int r = 0; r < RM; ++r) acc[r] = 0.f;
-
-  for (uint32_t k0 = 0; k0 < p.k; k0 += kBmmDepth) {
-    const uint32_t kc = min(kBmmDepth, p.k - k0);
-    // all staging loads in flight at once: clamped addresses, then predicated
-    // LDS stores
-    constexpr uint32_t kAPer = (TM * kBmmDepth + kBmmThreads - 1) / kBmmThreads;
-    _Float16 av[kAPer], bv[kBPer];
-#pragma unroll
-    for (uint32_t s = 0; s < kAPer; ++s) {
-      const uint32_t e = min(tid + s * kBmmThreads, TM * kBmmDepth - 1);
-      const uint32_t kk = p.a_kfast ? e % kBmmDepth : e / TM;
-      const uint32_t ii = p.a_kfast ? e / kBmmDepth : e % TM;
-      av[s] = p.a.p[p.a.at(bt, min(i0 + ii, p.m - 1), k0 + min(kk, kc - 1))];
-    }
-#pragma unroll
-    for (uint32_t s = 0; s < kBPer; ++s) {
-      const uint32_t e = tid + s * kBmmThreads;
-      const uint32_t kk = p.b_kfast ? e % kBmmDepth : e / kBmmCols;
-      bv[s] = p.b.p[bcol[s] + p.b.row.at(k0 + min(kk, kc - 1) + p.b.row_origin + bt * p.b.row_group)];
-    }
-#pragma unroll
-    for (uint32_t s = 0; s < kAPer; ++s) {
-      const uint32_t e = tid + s * kBmmThreads;
-      const uint32_t kk = p.a_kfast ? e % kBmmDepth : e / TM;
-      const uint32_t ii = p.a_kfast ? e / kBmmDepth : e % TM;
-      if (e < TM * kBmmDepth && kk < kc) As[kk][ii] = (float)av[s];
-    }
-#pragma unroll
-    for (uint32_t s = 0; s < kBPer; ++s) {
-      const uint32_t e = tid + s * kBmmThreads;
-      const uint32_t kk = p.b_kfast ? e % kBmmDepth : e / kBmmCols;
-      const uint32_t jj = p.b_kfast ? e / kBmmDepth : e % kBmmCols;
-      if (kk < kc) Bs[kk][jj] = (float)bv[s];
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (uint32_t kk = 0; kk < kc; ++kk) {
-      const float bv = Bs[kk][lane];
-#pragma unroll
-      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[kk][wave * RM + r], bv, acc[r]);
-    }
-    __syncthreads();
-  }
-  const uint32_t j = j0 + lane;
-  if (j >= p.n) return;
-#pragma unroll
-  for (int r = 0; r < RM; ++r) {
-    const uint32_t i = i0 + wave * RM + r;
-    if (i < p.m) p.y.p[p.y.at(bt, i, j)] = (_Float16)acc[r];
-  }
-}
-
-// ---------------------------------------------------------------- streamed b
-// When b holds every output column contiguously along k in 16-byte aligned
-// runs of 8 or more elements (the probabilities of v p^T, the blocked keys of
-// q^T k), lane j owns output column j and streams that column from memory with
-// 16-byte loads: b needs no LDS and no block-wide staging.  A block is one
-// wave; it stages its RM rows of a in LDS as fp32 (KS * 64 steps at a time)
-// and each reduction step is RM fmas on LDS broadcasts.  The column is read in
-// rounds of RV vectors (8 steps each): the first round is issued before the
-// rows of a are staged, each later round loads while the previous one is
-// consumed, and a whole round is consumed by straight-line code so that the
-// LDS reads of one vector overlap the fmas of the previous one.  KS and RV
-// are sized to K so that short reductions issue no surplus loads.
-template <int RM, int KS, int RV>
-__global__ __launch_bounds__(64) void bmm_stream_kernel(BmmPlan p) {
-  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-  constexpr uint32_t kDepth = KS * 64;  // steps of a staged per round (a multiple of 8 * RV)
-  __shared__ __attribute__((aligned(16))) float As[RM][kDepth];
-  const uint32_t lane = threadIdx.x;
-  uint32_t t = blockIdx.x;
-  const uint32_t q = p.div_nt.div(t), nt = t - q * p.ntiles;  // no integer division sequence
-  const uint32_t bt = p.div_mt.div(q), mt = q - bt * p.mtiles;
-  const uint32_t i0 = mt * RM, j = nt * kBmmCols + lane;
-  const _Float16* bcol = p.b.p + (int64_t)bt * p.b.batch +
-                         p.b.col.at(min(j, p.n - 1) + p.b.col_origin + bt * p.b.col_group);
-  const uint32_t rbase = p.b.row_origin + bt * p.b.row_group;
-  // vector v of the column holds steps [8v, 8v + 8).  Loads go through a
-  // buffer resource: the lane's column start is the vector offset, the step
-  // offset is uniform (a scalar register) and advances by 16 bytes per vector
-  // plus the run jump at each run end, so addressing costs a few scalar
-  // operations per vector.  Loads past the last whole vector re-read it and
-  // are not consumed.
-  const uint32_t nvec = p.k / 8;
-  const __amdgpu_buffer_rsrc_t brsrc = dev::buffer_rsrc(p.b.p, p.b_bytes);
-  const uint32_t bvoff = (uint32_t)(bcol - p.b.p) * 2u;
-  uint32_t bsoff = (uint32_t)p.b.row.at(rbase) * 2u;
-  uint32_t rpos = p.b_vrun ? (rbase - p.b.row.blk.div(rbase) * p.b.row.blk.d) / 8u : 0u;
-  uint32_t vaddr = 0;  // vector whose offset bsoff holds
-  auto load_round = [&](h8 (&buf)[RV]) {
-#pragma unroll
-    for (int v = 0; v < RV; ++v) {
-      buf[v] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bvoff, bsoff, 0));
-      if (vaddr + 1 < nvec) {
-        ++vaddr;
-        bsoff += 16u;
-        if (p.b_vrun && ++rpos == p.b_vrun) {
-          rpos = 0;
-          bsoff += p.b_vjump;
-        }
-      }
-    }
-  };
-  h8 cur[RV], nxt[RV];
-  if (nvec) load_round(cur);
-
-  float acc[RM];
-#pragma unroll
-  for (int r = 0; r < RM; ++r) acc[r] = 0.f;
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  // rows' steps kk..kk+7 of the staged a
-  auto read_a = [&](f4 (&a)[RM][2], uint32_t kk) {
-#pragma unroll
-    for (int r = 0; r < RM; ++r) {
-      a[r][0] = *reinterpret_cast<const f4*>(&As[r][kk]);
-      a[r][1] = *reinterpret_cast<const f4*>(&As[r][kk + 4]);
-    }
-  };
-  auto fmas = [&](const f4 (&a)[RM][2], const h8& v) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float bv = (float)v[q];
-#pragma unroll
-      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(a[r][q / 4][q % 4], bv, acc[r]);
-    }
-  };
-  auto consume = [&](const h8& v, uint32_t kk) {
-    f4 a[RM][2];
-    read_a(a, kk);
-    fmas(a, v);
-  };
-  uint32_t vnext = 0;  // first vector not yet consumed (a multiple of RV between rounds)
-  for (uint32_t k0 = 0; k0 < p.k; k0 += kDepth) {
-    const uint32_t kc = min(kDepth, p.k - k0);
-    if (k0) __syncthreads();  // the previous round's rows are no longer read
-    {
-      // every load of the round in flight at once: clamped addresses, then
-      // predicated LDS stores
-      int64_t colpart[KS];
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        colpart[s] = p.a.col.at(k0 + min(lane + s * 64u, kc - 1) + p.a.col_origin + bt * p.a.col_group);
-      _Float16 av[RM][KS];
-#pragma unroll
-      for (int r = 0; r < RM; ++r) {
-        const _Float16* row = p.a.p + (int64_t)bt * p.a.batch +
-                              p.a.row.at(min(i0 + r, p.m - 1) + p.a.row_origin + bt * p.a.row_group);
-#pragma unroll
-        for (int s = 0; s < KS; ++s) av[r][s] = row[colpart[s]];
-      }
-#pragma unroll
-      for (int r = 0; r < RM; ++r)
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-          if (lane + s * 64u < kc) As[r][lane + s * 64] = (float)av[r][s];
-    }
-    __syncthreads();
-    const uint32_t vend = min(nvec, (k0 + kc) / 8);  // whole vectors inside this round
-    // whole rounds: straight-line code
-    while (vnext + RV <= vend) {
-      const bool more = vnext + RV < nvec;
-      if (more) load_round(nxt);
-      // the a steps of vector v + 1 are read while vector v's fmas run
-      f4 a0[RM][2], a1[RM][2];
-      const uint32_t kb = vnext * 8 - k0;
-      read_a(a0, kb);
-#pragma unroll
-      for (int v = 0; v < RV; v += 2) {
-        read_a(a1, kb + (v + 1) * 8);
-        fmas(a0, cur[v]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (v + 2 < RV) read_a(a0, kb + (v + 2) * 8);
-        fmas(a1, cur[v + 1]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (more) {
-#pragma unroll
-        for (int v = 0; v < RV; ++v) cur[v] = nxt[v];
-      }
-      vnext += RV;
-    }
-    // the last, partial round
-    if (vnext < vend) {
-#pragma unroll
-      for (int v = 0; v < RV; ++v)
-        if (vnext + v < vend) consume(cur[v], (vnext + v) * 8 - k0);
-      vnext = vend;
-    }
-    // steps past the last whole vector
-    for (uint32_t kk = max(k0, nvec * 8); kk < k0 + kc; ++kk) {
-      const float bv = (float)bcol[p.b.row.at(rbase + kk)];
-#pragma unroll
-      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[r][kk - k0], bv, acc[r]);
-    }
-  }
-  if (j >= p.n) return;
-#pragma unroll
-  for (int r = 0; r < RM; ++r) {
-    const uint32_t i = i0 + r;
-    if (i < p.m) p.y.p[p.y.at(bt, i, j)] = (_Float16)acc[r];
-  }
-}
-
-template <int RM>
-void launch_stream(const BmmPlan& p, uint32_t grid, hipStream_t stream) {
-  if (p.k <= 32)
-    hipLaunchKernelGGL((bmm_stream_kernel<RM, 1, 4>), dim3(grid), dim3(64), 0, stream, p);
-  else if (p.k <= 64)
-    hipLaunchKernelGGL((bmm_stream_kernel<RM, 1, 8>), dim3(grid), dim3(64), 0, stream, p);
-  else
-    hipLaunchKernelGGL((bmm_stream_kernel<RM, 8, 8>), dim3(grid), dim3(64), 0, stream, p);
-}
-
-// ---------------------------------------------------------------- tiled b
-// b streamable as above but with columns at least a cache line apart (the
-// probabilities of v p^T: each column is a row of p): a lane that streams its
-// own column touches a different line per lane and instruction, which
-// saturates the L1 tag lookups.  Here a block of 4 waves computes 4 * RM rows
-// x 64 columns and loads b in kTileDepth-step chunks with 8 lanes per column
-// (one 128-byte line per 8 lanes), keeps them in LDS as fp16 step pairs, and
-// each lane reads its column two steps at a time (one 32-bit LDS read for two
-// fmas; the fp16 -> fp32 conversion folds into the fma).  The next chunk is
-// loaded into registers while the current one is consumed.  K % 8 == 0.
+// The f32 matrix instruction shares its issue with the VALU (each VALU
+// instruction between two of them costs about 8 cycles; one takes 32), so the
+// loops hold as little else as they can: operands are widened to fp32 once, on
+// their way into LDS (widening each lane's operands in the loop instead: 111
+// of 140 TFLOP/s in a loop of products alone), the loads take a scalar base
+// and a lane offset that stays the same from chunk to chunk, and LDS buffers
+// are compile-time offsets.
 //
-// Each output is a chain of K dependent fmas, and a dependent fp32 fma takes
-// about 32 cycles on gfx950 (measured), so a K = 400 product cannot finish in
-// under ~5.6 us however it is tiled; the tile shape only has to keep every
-// chain running.
-constexpr uint32_t kTileDepth = 64;
+// Staging of one operand's R rows x KD steps.  Every load is a 16-byte run of
+// 8 steps of a row or 8 rows of a step (any 2-byte alignment) at an address
+// clamped into the operand, with no branch around it, so that all of a chunk's
+// loads are in flight at once.
+//
+// Step-major operands (RF false: the steps of a row are adjacent in memory)
+// lie in LDS per 32 steps as [row][8 slots][4 floats]: the instruction's lane
+// (i, g) takes step 4s + g of row i in its s-th call, so calls 4h..4h+3 are
+// slot (h, g), one 16-byte read.  Slot h is swapped by bit 1 of the row and g
+// xored with minus the row's group of four, which puts each 16 lanes that a
+// 16-byte read serves at once (0-3, 12-15, 20-27; 4-11, 16-19, 28-31) on
+// distinct banks; 32-step groups are one slot apart for the writes.
+// Row-major operands (RF true: the rows of a step are adjacent) lie
+// [step][row], a lane reading its W adjacent rows of one step at a time; half
+// a row group is swapped for alternate steps (W = 2) or step pairs (W = 1),
+// so that the four steps of a call lie on distinct banks.
+//
+// SECOND: an operand of fewer units than threads takes the upper threads.
+template <bool RF, int KD, int R, int W, bool SECOND = false>
+struct Stage {
+  static constexpr uint32_t kGroup = R * 32 + 4;                     // !RF: floats per 32 steps
+  static constexpr uint32_t kFloats = RF ? KD * R : KD / 32 * kGroup;
+  static constexpr uint32_t kUnits = RF ? KD * R / 8 : KD * R / 16;  // a run of 8 / two runs of 8 steps
+  static constexpr uint32_t kPer = kUnits < kBmmThreads ? 1 : kUnits / kBmmThreads;
+  static constexpr uint32_t kAcross = RF ? R / 8 : KD / 16;          // units side by side along the memory axis
+  static constexpr uint32_t kNext = kBmmThreads / kAcross;           // steps between a thread's units
+  static_assert(RF || kPer == 1, "one unit of a step-major operand per thread");
+  static constexpr uint32_t kLoads = RF ? kPer : 2;
 
-template <int RM>
-__global__ __launch_bounds__(kBmmThreads) void bmm_tile_kernel(BmmPlan p) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-  constexpr uint32_t TM = 4 * RM;
-  constexpr uint32_t kAPitch = TM + 4;
-  constexpr uint32_t kBPitch = kBmmCols + 1;  // in step pairs
-  constexpr uint32_t kAPer = TM * kTileDepth / kBmmThreads;  // a elements per thread per chunk
-  __shared__ __attribute__((aligned(16))) float As[kTileDepth][kAPitch];
-  __shared__ h2 Bs[kTileDepth / 2][kBPitch];
+  uint32_t off[kLoads];            // bytes from the base of the batch entry
+  uint32_t to[RF ? 1 : 4];         // LDS position (floats)
+  using Regs = h8[kLoads];
+
+  static __device__ __forceinline__ uint32_t tid() {
+    return SECOND && kUnits < kBmmThreads ? threadIdx.x ^ (kBmmThreads / 2) : threadIdx.x;
+  }
+  static __device__ __forceinline__ bool active() { return kUnits >= kBmmThreads || tid() < kUnits; }
+  static __device__ __forceinline__ uint32_t across() { return tid() % kAcross; }
+  // the row (step) of the thread's unit: 32-step chunks, two units to a row,
+  // deal rows 1, 8 and 16 apart to neighbouring threads, whose LDS writes then
+  // fall on distinct banks
+  static __device__ __forceinline__ uint32_t along() {
+    const uint32_t a = tid() / kAcross;
+    if (RF || KD != 32) return a;
+    return (a & 33u) | (a & 6u) << 2 | (a & 24u) >> 2;
+  }
+  static __device__ __forceinline__ uint32_t slot(uint32_t row, uint32_t h, uint32_t g) {
+    return row * 32u + ((h ^ (row >> 1 & 1u)) * 4u + (g ^ ((0u - row / (4u * W)) & 3u))) * 4u;
+  }
+  static __device__ __forceinline__ uint32_t swapped(uint32_t step, uint32_t row) {  // RF: place in the step
+    return W == 2 ? row ^ (step & 1u) * 32u : row ^ (step >> 1 & 1u) * 16u;
+  }
+
+  static __device__ __forceinline__ const char* base(const Side& s, uint32_t bt) {
+    return reinterpret_cast<const char*>(s.p + (int64_t)bt * s.batch);
+  }
+
+  __device__ __forceinline__ void place() {
+    if constexpr (RF) {
+      to[0] = along() * R + swapped(along(), across() * 8u);  // kNext is a multiple of 4
+    } else {
+#pragma unroll
+      for (uint32_t g = 0; g < 4; ++g) to[g] = across() / 2 * kGroup + slot(along(), across() & 1u, g);
+    }
+  }
+
+  // offsets of the tile from row r0 and step k0
+  __device__ __forceinline__ void aim(const Side& s, uint32_t bt, uint32_t r0, uint32_t k0, uint32_t K) {
+    const uint32_t ro = s.row_origin + bt * s.row_group, so = s.step_origin + bt * s.step_group;
+    if constexpr (RF) {
+      const int64_t row = s.row.at(ro + min(r0 + across() * 8u, s.rows - 8u));
+#pragma unroll
+      for (uint32_t u = 0; u < kPer; ++u)
+        off[u] = (uint32_t)(row + s.step.at(so + min(k0 + along() + u * kNext, K - 1u))) * 2u;
+    } else {
+      const int64_t row = s.row.at(ro + min(r0 + along(), s.rows - 1u));
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h)
+        off[h] = (uint32_t)(row + s.step.at(so + min(k0 + across() * 16u + 8u * h, K - 8u))) * 2u;
+    }
+  }
+
+  __device__ __forceinline__ void load(const char* b, Regs& v) {
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; ++u) {
+      __asm__("" : "+v"(off[u]));  // keeps the offset 32 bits wide: one scalar base and one register a load
+      v[u] = *reinterpret_cast<const h8u*>(b + off[u]);
+    }
+  }
+
+  // zeroes the steps past the end (a zero product leaves every sum as it is);
+  // the run of steps across the end was loaded as the last 8
+  __device__ __forceinline__ void trim(uint32_t k0, uint32_t K, Regs& v) const {
+    const h8 zero = (h8)(_Float16)0;
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; ++u) {
+      if constexpr (RF) {
+        if (k0 + along() + u * kNext >= K) v[u] = zero;
+      } else {
+        typedef uint64_t u2 __attribute__((ext_vector_type(2)));
+        const uint32_t k = k0 + across() * 16u + 8u * u, c = K & 7u, cut = 16u * (8u - c);
+        if (c && k < K && k + 8u > K) {
+          const u2 d = __builtin_bit_cast(u2, v[u]);
+          const u2 r = cut < 64u ? (u2){d[0] >> cut | d[1] << (64u - cut), d[1] >> cut} : (u2){d[1] >> (cut - 64u), 0};
+          v[u] = __builtin_bit_cast(h8, r);
+        }
+        if (k >= K) v[u] = zero;
+      }
+    }
+  }
+
+  __device__ __forceinline__ void store(float* lds, const Regs& v) const {
+    if (!active()) return;
+    if constexpr (RF) {
+#pragma unroll
+      for (uint32_t u = 0; u < kPer; ++u) {
+        f4* d = reinterpret_cast<f4*>(lds + to[0] + u * kNext * R);
+        d[0] = (f4){(float)v[u][0], (float)v[u][1], (float)v[u][2], (float)v[u][3]};
+        d[1] = (f4){(float)v[u][4], (float)v[u][5], (float)v[u][6], (float)v[u][7]};
+      }
+    } else {
+#pragma unroll
+      for (uint32_t g = 0; g < 4; ++g)
+        *reinterpret_cast<f4*>(lds + to[g]) =
+            (f4){(float)v[0][g], (float)v[0][g + 4], (float)v[1][g], (float)v[1][g + 4]};
+    }
+  }
+
+  // tile row that instruction row i of the wave's tile t holds; the 4 rows a
+  // lane gets back, over the W tiles, are 4 * W consecutive ones either way
+  static __device__ __forceinline__ uint32_t row_of(uint32_t i, uint32_t t) {
+    return RF ? i * W + t : (i >> 2) * (4u * W) + 4u * t + (i & 3u);
+  }
+  // position of (instruction row r of 4, tile t) in those 4 * W rows
+  static __device__ __forceinline__ constexpr uint32_t place_of(uint32_t r, uint32_t t) { return RF ? r * W + t : 4u * t + r; }
+};
+
+// A wave's reads of W tiles of an operand, 8 calls (32 steps) at a time.
+template <bool RF, int KD, int R, int W>
+struct Operand {
+  using S = Stage<RF, KD, R, W>;
+  typedef float fw __attribute__((ext_vector_type(W)));
+  uint32_t at[RF ? 1 : 2 * W];
+  struct Group {
+    f4 steps[RF ? 1 : W][2];
+    fw rows[RF ? 8 : 1];
+    __device__ __forceinline__ float value(uint32_t s, uint32_t t) const {
+      if constexpr (RF) return rows[s][t];
+      else return steps[t][s / 4][s % 4];
+    }
+  };
+
+  __device__ __forceinline__ void init(uint32_t wave_row, uint32_t lane) {
+    const uint32_t i = lane & 15u, g = lane >> 4;
+    if constexpr (RF) {
+      at[0] = g * R + S::swapped(g, wave_row + i * W);
+    } else {
+#pragma unroll
+      for (uint32_t t = 0; t < W; ++t)
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) at[2 * t + h] = S::slot(wave_row + S::row_of(i, t), h, g);
+    }
+  }
+  __device__ __forceinline__ void read(Group& d, const float* lds, uint32_t c32) const {
+    if constexpr (RF) {
+#pragma unroll
+      for (uint32_t s = 0; s < 8; ++s) d.rows[s] = *reinterpret_cast<const fw*>(lds + at[0] + (c32 * 32u + 4u * s) * R);
+    } else {
+#pragma unroll
+      for (uint32_t t = 0; t < W; ++t)
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h)
+          d.steps[t][h] = *reinterpret_cast<const f4*>(lds + at[2 * t + h] + c32 * S::kGroup);
+    }
+  }
+};
+
+// FIRST: from zero sums
+template <int W, bool FIRST = false, class GP, class GQ>
+__device__ __forceinline__ void bmm_call(f4 (&acc)[W][W], const GP& gp, const GQ& gq, uint32_t s) {
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(gp.value(s, i), gq.value(s, j),
+                                                       FIRST ? (f4){0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
+}
+
+// The wave's outputs: p index pr holds the lane's first, rows below plo / qlo
+// belong to another block.
+template <int W, class SP, class SQ>
+__device__ __forceinline__ void bmm_write(const BmmPlan& p, uint32_t bt, const f4 (&acc)[W][W], uint32_t pr, uint32_t plo,
+                                          uint32_t q0, uint32_t qlo, uint32_t lane) {
+  _Float16* y = p.y + (int64_t)bt * p.ybatch;
+  const uint32_t po = pr + bt * p.yp_group;
+#pragma unroll
+  for (uint32_t t = 0; t < W; ++t) {
+    const uint32_t q = q0 + SQ::row_of(lane & 15u, t);
+    if (q >= p.Q.rows || q < qlo) continue;
+    typedef _Float16 hv __attribute__((ext_vector_type(4 * W), aligned(2)));
+    hv o;
+#pragma unroll
+    for (uint32_t a = 0; a < W; ++a)
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) o[SP::place_of(r, a)] = (_Float16)acc[a][t][r];
+    _Float16* row = y + p.yq.at(q);
+    if (p.y_vec && pr >= plo && pr + 4u * W <= p.P.rows) {
+      *reinterpret_cast<hv*>(row + p.yp.at(po)) = o;
+    } else {
+#pragma unroll
+      for (uint32_t e = 0; e < 4 * W; ++e)
+        if (pr + e >= plo && pr + e < p.P.rows) row[p.yp.at(po + e)] = o[e];
+    }
+  }
+}
+
+// First row of a tile: the last tile of a row-major operand whose rows are no
+// multiple of 8 starts up to 7 rows early, so that its rows are whole runs
+// (the rows it shares with the tile before are not written).
+template <bool RF>
+__device__ __forceinline__ uint32_t tile_row(uint32_t tile, uint32_t tiles, uint32_t r, uint32_t rows) {
+  return RF && tile + 1u == tiles ? tile * r - ((0u - rows) & 7u) : tile * r;
+}
+
+template <int B>
+struct Const {
+  static constexpr int value = B;
+};
+
+// y[p, q] = sum_k P[p, k] Q[q, k] for K > 32, a block of 4 waves per 32W x 32W
+// outputs, W x W instruction tiles per wave.  Chunks of KD steps alternate
+// between two LDS buffers; the loads of the next two chunks are in flight under
+// the products of this one (one: 41.2 against 36.4 us for the batched v p^T,
+// four: 40.7).
+//
+// Bound by the issue of the products and of the VALU work beside them: the
+// matrix pipe is busy 55-60% of the launch, at [128,64,400] x [128,400,400]
+// 36.4 us (72 TFLOP/s; 80.5 us with the fma chains this replaced) against the
+// 17 us that the products alone take at 153 TFLOP/s.
+template <int KD, int W, bool PR, bool QR>
+__global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPlan p) {
+  constexpr int R = 32 * W;
+  using SP = Stage<PR, KD, R, W>;
+  using SQ = Stage<QR, KD, R, W, true>;
+  using OP = Operand<PR, KD, R, W>;
+  using OQ = Operand<QR, KD, R, W>;
+  constexpr int PF = 2;
+  constexpr uint32_t kBuf = SP::kFloats + SQ::kFloats;
+  __shared__ __attribute__((aligned(16))) float lds[2 * kBuf];
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t rest = p.pblocks.div(blockIdx.x), pt = blockIdx.x - rest * p.pblocks.d;
+  const uint32_t bt = p.qtiles.div(rest), qt = rest - bt * p.qtiles.d;
+  const uint32_t K = p.k;
+  const uint32_t p0 = tile_row<PR>(pt, p.ptiles, R, p.P.rows), q0 = tile_row<QR>(qt, p.qtiles.d, R, p.Q.rows);
+  const uint32_t last = (K - 1u) / KD;  // the last chunk, whole or not
+
+  SP sp;
+  SQ sq;
+  typename SP::Regs vp[PF];
+  typename SQ::Regs vq[PF];
+  const char* bp = SP::base(p.P, bt);
+  const char* bq = SQ::base(p.Q, bt);
+  sp.aim(p.P, bt, p0, 0, K);
+  sq.aim(p.Q, bt, q0, 0, K);
+  uint32_t n = 0;  // the next chunk to load
+  // chunk n into register set n % PF; past the last chunk that one again,
+  // which nothing stores: a test around the loads would leave the waits
+  // without a count of the loads behind the one they wait for
+  auto load = [&](int set) __attribute__((always_inline)) {
+    if (n == last) {
+      sp.aim(p.P, bt, p0, last * KD, K);
+      sq.aim(p.Q, bt, q0, last * KD, K);
+      bp = SP::base(p.P, bt);
+      bq = SQ::base(p.Q, bt);
+    }
+    sp.load(bp, vp[set]);
+    sq.load(bq, vq[set]);
+    if (n < last) {
+      bp += p.P.hop;
+      bq += p.Q.hop;
+    }
+    ++n;
+  };
+#pragma unroll
+  for (int set = 0; set < PF; ++set) load(set);
+  sp.place();
+  sq.place();
+  const uint32_t wp = (wave & 1u) * 16u * W, wq = (wave >> 1) * 16u * W;  // the wave's rows in the tile
+  const bool work = p0 + wp < p.P.rows && q0 + wq < p.Q.rows;
+  OP op;
+  OQ oq;
+  op.init(wp, lane);
+  oq.init(wq, lane);
+  f4 acc[W][W];
+#pragma unroll
+  for (int a = 0; a < W; ++a)
+#pragma unroll
+    for (int b = 0; b < W; ++b) acc[a][b] = (f4){0.f, 0.f, 0.f, 0.f};
+
+  typename OP::Group gp[2];
+  typename OQ::Group gq[2];
+  uint32_t c = 0;  // the chunk to multiply
+  auto store = [&](int set, float* to, bool end) __attribute__((always_inline)) {
+    if (end) {
+      sp.trim(last * KD, K, vp[set]);
+      sq.trim(last * KD, K, vq[set]);
+    }
+    sp.store(to, vp[set]);
+    sq.store(to + SP::kFloats, vq[set]);
+  };
+  // chunk c = S mod PF from its buffer, chunk c + 1 into the other
+  auto step = [&](auto S) __attribute__((always_inline)) {
+    constexpr int set = decltype(S)::value;
+    constexpr uint32_t kFrom = set & 1 ? kBuf : 0, kTo = kBuf - kFrom;
+    load(set);
+    if (work) {
+      op.read(gp[0], lds + kFrom, 0);
+      oq.read(gq[0], lds + kFrom + SP::kFloats, 0);
+#pragma unroll
+      for (uint32_t g = 0; g < KD / 32; ++g) {
+        if (g + 1 < KD / 32) {  // the next 32 steps, under the products of these
+          op.read(gp[(g + 1) & 1], lds + kFrom, g + 1);
+          oq.read(gq[(g + 1) & 1], lds + kFrom + SP::kFloats, g + 1);
+        }
+#pragma unroll
+        for (uint32_t s = 0; s < 8; ++s) bmm_call<W>(acc, gp[g & 1], gq[g & 1], s);
+      }
+    }
+    ++c;
+    // every wave was done with that buffer's chunk c - 1 at the last barrier
+    store((set + 1) % PF, lds + kTo, c == last);
+    __syncthreads();
+    return c < last;
+  };
+  store(0, lds, last == 0);
+  __syncthreads();
+  if (last) {
+    while (step(Const<0>()) && step(Const<1>())) {
+    }
+  }
+  if (!work) return;
+  const float* from = lds + (last & 1u ? kBuf : 0u);
+  uint32_t calls = (K - last * KD + 3u) / 4u;
+  for (uint32_t g = 0; calls; ++g) {
+    op.read(gp[0], from, g);
+    oq.read(gq[0], from + SP::kFloats, g);
+    if (calls >= 8u) {
+#pragma unroll
+      for (uint32_t s = 0; s < 8; ++s) bmm_call<W>(acc, gp[0], gq[0], s);
+      calls -= 8u;
+    } else {
+#pragma unroll
+      for (uint32_t s = 0; s < 7; ++s)
+        if (s < calls) bmm_call<W>(acc, gp[0], gq[0], s);
+      calls = 0;
+    }
+  }
+  bmm_write<W, SP, SQ>(p, bt, acc, p0 + wp + (lane >> 4) * (4u * W), pt * R, q0 + wq, qt * R, lane);
+}
+
+// The same for K <= 32 (one chunk): the block keeps its Q operand in registers
+// and walks `span` P tiles, the next tile's loads in flight under the products
+// and stores of this one.  At [128,400,32] x [128,32,400] 24.3 us (96.9 with
+// the fma chains this replaced), where the products take 9 us and the 41 MB
+// of outputs about 8.
+template <int W, bool PR, bool QR>
+__global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
+  constexpr int KD = 32, R = 32 * W;
+  using SP = Stage<PR, KD, R, W>;
+  using SQ = Stage<QR, KD, R, W, true>;
+  using OP = Operand<PR, KD, R, W>;
+  using OQ = Operand<QR, KD, R, W>;
+  __shared__ __attribute__((aligned(16))) float lds[SQ::kFloats + 2 * SP::kFloats];
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t rest = p.pblocks.div(blockIdx.x), pb = blockIdx.x - rest * p.pblocks.d;
+  const uint32_t bt = p.qtiles.div(rest), qt = rest - bt * p.qtiles.d;
+  const uint32_t K = p.k;
+  const uint32_t q0 = tile_row<QR>(qt, p.qtiles.d, R, p.Q.rows);
+  uint32_t pt = pb * p.span;
+  const uint32_t pend = min(pt + p.span, p.ptiles);
+
+  SP sp;
+  SQ sq;
+  typename SP::Regs vp;
+  typename SQ::Regs vq;
+  const char* bp = SP::base(p.P, bt);
+  uint32_t p0 = tile_row<PR>(pt, p.ptiles, R, p.P.rows);
+  sp.aim(p.P, bt, p0, 0, K);
+  sq.aim(p.Q, bt, q0, 0, K);
+  sq.load(SQ::base(p.Q, bt), vq);
+  sp.load(bp, vp);
+  sp.place();
+  sq.place();
+  const uint32_t wp = (wave & 1u) * 16u * W, wq = (wave >> 1) * 16u * W;
+  OP op;
+  OQ oq;
+  op.init(wp, lane);
+  oq.init(wq, lane);
+  float* const ldsp = lds + SQ::kFloats;
+  if (K < KD) {
+    sq.trim(0, K, vq);
+    sp.trim(0, K, vp);
+  }
+  sq.store(lds, vq);
+  sp.store(ldsp, vp);
+  __syncthreads();
+  typename OQ::Group gq;
+  oq.read(gq, lds, 0);
+  const uint32_t calls = (K + 3u) / 4u;
+  // the lane's outputs of a whole tile: one run of 4 * W per q row
+  typedef _Float16 hv __attribute__((ext_vector_type(4 * W), aligned(2)));
+  _Float16* out[W];
+  bool mine[W];
+#pragma unroll
+  for (uint32_t t = 0; t < W; ++t) {
+    const uint32_t q = q0 + wq + SQ::row_of(lane & 15u, t);
+    mine[t] = q < p.Q.rows && q >= qt * R;
+    out[t] = p.y + ((int64_t)bt * p.ybatch + p.yq.at(min(q, p.Q.rows - 1u)) +
+                    p.yp.at(pt * R + wp + (lane >> 4) * (4u * W) + bt * p.yp_group));
+  }
+  auto step = [&](auto B) __attribute__((always_inline)) {  // tile pt from buffer B, the next one into the other
+    constexpr uint32_t kFrom = decltype(B)::value ? SP::kFloats : 0, kTo = SP::kFloats - kFrom;
+    const bool more = pt + 1u < pend;
+    const uint32_t pr = p0 + wp;
+    if (more) {
+      p0 = tile_row<PR>(pt + 1u, p.ptiles, R, p.P.rows);
+      if (pt + 2u == p.ptiles) {
+        sp.aim(p.P, bt, p0, 0, K);
+        bp = SP::base(p.P, bt);
+      } else {
+        bp += p.P.hop;
+      }
+      sp.load(bp, vp);
+    }
+    if (pr < p.P.rows && q0 + wq < p.Q.rows) {
+      typename OP::Group gp;
+      op.read(gp, ldsp + kFrom, 0);
+      f4 acc[W][W];
+      bmm_call<W, true>(acc, gp, gq, 0);
+      if (calls == 8u) {
+#pragma unroll
+        for (uint32_t s = 1; s < 8; ++s) bmm_call<W>(acc, gp, gq, s);
+      } else {
+#pragma unroll
+        for (uint32_t s = 1; s < 7; ++s)
+          if (s < calls) bmm_call<W>(acc, gp, gq, s);
+      }
+      if (p.y_vec && pt + 1u < p.ptiles) {
+#pragma unroll
+        for (uint32_t t = 0; t < W; ++t) {
+          hv o;
+#pragma unroll
+          for (uint32_t a = 0; a < W; ++a)
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) o[SP::place_of(r, a)] = (_Float16)acc[a][t][r];
+          if (mine[t]) *reinterpret_cast<hv*>(out[t]) = o;
+          out[t] += p.yhop;
+        }
+      } else {
+        bmm_write<W, SP, SQ>(p, bt, acc, pr + (lane >> 4) * (4u * W), pt * R, q0 + wq, qt * R, lane);
+      }
+    }
+    if (more) {
+      if (K < KD) sp.trim(0, K, vp);
+      sp.store(ldsp + kTo, vp);
+      __syncthreads();
+    }
+    ++pt;
+  };
+  for (;;) {
+    step(Const<0>());
+    if (pt >= pend) break;
+    step(Const<1>());
+    if (pt >= pend) break;
+  }
+}
+
+// Steps per chunk of bmm_kernel, measured on v p^T: the 64 x 64 form, with
+// three or four blocks on a compute unit, takes 36.4 us with 32 at
+// [128,64,400] x [128,400,400] and 39.2 with 64; the 32 x 32 form, with one or
+// two, 21.7 us with 128 at [4,64,1600] x [4,1600,1600] and 23.7 with 64.
+constexpr int bmm_depth(int w) { return w == 2 ? 32 : 128; }
+
+// Any strides: the elements are gathered, 32 steps a chunk, into [step][row]
+// tiles of RP and RQ rows (RP * RQ = 1024), one 16 x 16 instruction tile per
+// wave.  Bound by the element loads and their addresses, so an operand of at
+// most 16 rows takes a tile of 16 ([128,8,400] x [128,400,400], both of stride
+// 2: 46 us with 32); every load is in range by its clamped index (under a
+// test, each waits for the one before: 1.5x), and 64-step chunks measured
+// 1.1-1.8x slower.
+template <int RP, int RQ>
+__global__ __launch_bounds__(kBmmThreads) void bmm_gather_kernel(BmmPlan p) {
+  constexpr int KD = 32;
+  static_assert(RP * RQ == 1024, "one 16 x 16 tile for each of 4 waves");
+  __shared__ float ldsp[KD * (RP + 1)], ldsq[KD * (RQ + 1)];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  uint32_t t = blockIdx.x;
-  const uint32_t nt = t % p.ntiles;
-  t /= p.ntiles;
-  const uint32_t mt = t % p.mtiles;
-  const uint32_t bt = t / p.mtiles;
-  const uint32_t i0 = mt * TM, j0 = nt * kBmmCols;
-
-  // b: thread handles vectors e = tid + 256 s: column jj = e / 8, steps
-  // 8 * (e % 8) .. + 8 of the chunk
-  const __amdgpu_buffer_rsrc_t brsrc = dev::buffer_rsrc(p.b.p, p.b_bytes);
-  const uint32_t rbase = p.b.row_origin + bt * p.b.row_group;
-  uint32_t bvoff[2];
+  const uint32_t rest = p.pblocks.div(blockIdx.x), pt = blockIdx.x - rest * p.pblocks.d;
+  const uint32_t bt = p.qtiles.div(rest), qt = rest - bt * p.qtiles.d;
+  const uint32_t K = p.k;
+  _Float16 vp[RP * KD / kBmmThreads], vq[RQ * KD / kBmmThreads];
+  auto load = [&](auto R, const Side& s, uint32_t tile, uint32_t k0, auto& d) __attribute__((always_inline)) {
+    const _Float16* src = s.p + (int64_t)bt * s.batch;
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const uint32_t jj = (tid + s * kBmmThreads) / 8u;
-    bvoff[s] = (uint32_t)((int64_t)bt * p.b.batch +
-                          p.b.col.at(min(j0 + jj, p.n - 1) + p.b.col_origin + bt * p.b.col_group)) * 2u;
-  }
-  const uint32_t kv = tid % 8u;
-  h8 bv[2];
-  _Float16 av[kAPer];
-  auto load_chunk = [&](uint32_t k0, uint32_t kc) {
-    // vectors past the chunk's end re-read its last vector (never consumed)
-    const uint32_t kk = k0 + min(kv * 8u, kc - 8u);
-    const uint32_t soff = (uint32_t)p.b.row.at(rbase + kk) * 2u;
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-      bv[s] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bvoff[s] + soff, 0, 0));
-#pragma unroll
-    for (uint32_t s = 0; s < kAPer; ++s) {
-      const uint32_t e = tid + s * kBmmThreads;
-      const uint32_t kk2 = p.a_kfast ? e % kTileDepth : e / TM;
-      const uint32_t ii = p.a_kfast ? e / kTileDepth : e % TM;
-      av[s] = p.a.p[p.a.at(bt, min(i0 + ii, p.m - 1), k0 + min(kk2, kc - 1))];
+    for (uint32_t u = 0; u < sizeof(d) / 2; ++u) {
+      const uint32_t e = tid + u * kBmmThreads;
+      const uint32_t r = s.steps_near ? e / KD : e % R.value, k = s.steps_near ? e % KD : e / R.value;
+      d[u] = src[s.row.at(s.row_origin + bt * s.row_group + min(tile * R.value + r, s.rows - 1u)) +
+                 s.step.at(s.step_origin + bt * s.step_group + min(k0 + k, K - 1u))];
     }
   };
-  auto store_chunk = [&]() {
+  auto store = [&](auto R, const Side& s, uint32_t k0, const auto& d, float* to) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const uint32_t jj = (tid + s * kBmmThreads) / 8u;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) Bs[kv * 4 + q][jj] = (h2){bv[s][2 * q], bv[s][2 * q + 1]};
-    }
-#pragma unroll
-    for (uint32_t s = 0; s < kAPer; ++s) {
-      const uint32_t e = tid + s * kBmmThreads;
-      const uint32_t kk2 = p.a_kfast ? e % kTileDepth : e / TM;
-      const uint32_t ii = p.a_kfast ? e / kTileDepth : e % TM;
-      As[kk2][ii] = (float)av[s];
+    for (uint32_t u = 0; u < sizeof(d) / 2; ++u) {
+      const uint32_t e = tid + u * kBmmThreads;
+      const uint32_t r = s.steps_near ? e / KD : e % R.value, k = s.steps_near ? e % KD : e / R.value;
+      to[k * (R.value + 1) + r] = k0 + k < K ? (float)d[u] : 0.f;  // zero steps past the end leave the sums as they are
     }
   };
-
-  float acc[RM];
-#pragma unroll
-  for (int r = 0; r < RM; ++r) acc[r] = 0.f;
-  load_chunk(0, min(kTileDepth, p.k));
-  for (uint32_t k0 = 0; k0 < p.k; k0 += kTileDepth) {
-    const uint32_t kc = min(kTileDepth, p.k - k0);
-    store_chunk();
+  const uint32_t i = lane & 15u, g = lane >> 4, wp = wave % (RP / 16) * 16u, wq = wave / (RP / 16) * 16u;
+  f4 acc[1][1] = {{(f4){0.f, 0.f, 0.f, 0.f}}};
+  load(Const<RP>(), p.P, pt, 0, vp);
+  load(Const<RQ>(), p.Q, qt, 0, vq);
+  for (uint32_t k0 = 0; k0 < K; k0 += KD) {
+    if (k0) __syncthreads();
+    store(Const<RP>(), p.P, k0, vp, ldsp);
+    store(Const<RQ>(), p.Q, k0, vq, ldsq);
     __syncthreads();
-    if (k0 + kTileDepth < p.k) load_chunk(k0 + kTileDepth, min(kTileDepth, p.k - k0 - kTileDepth));
-#pragma unroll 4
-    for (uint32_t k2 = 0; k2 < kc / 2; ++k2) {
-      const h2 b = Bs[k2][lane];
-      const float b0 = (float)b[0], b1 = (float)b[1];
-#pragma unroll
-      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[2 * k2][wave * RM + r], b0, acc[r]);
-#pragma unroll
-      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[2 * k2 + 1][wave * RM + r], b1, acc[r]);
+    if (k0 + KD < K) {
+      load(Const<RP>(), p.P, pt, k0 + KD, vp);
+      load(Const<RQ>(), p.Q, qt, k0 + KD, vq);
     }
-    __syncthreads();
-  }
-  const uint32_t j = j0 + lane;
-  if (j >= p.n) return;
 #pragma unroll
-  for (int r = 0; r < RM; ++r) {
-    const uint32_t i = i0 + wave * RM + r;
-    if (i < p.m) p.y.p[p.y.at(bt, i, j)] = (_Float16)acc[r];
+    for (uint32_t s = 0; s < KD / 4; ++s)
+      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ldsp[(4 * s + g) * (RP + 1) + wp + i],
+                                                       ldsq[(4 * s + g) * (RQ + 1) + wq + i], acc[0][0], 0, 0, 0);
   }
+  using S = Stage<false, 32, 32, 1>;
+  bmm_write<1, S, S>(p, bt, acc, pt * RP + wp + g * 4u, pt * RP, qt * RQ + wq, qt * RQ, lane);
+}
+
+template <bool SHORT, int W, bool PR, bool QR>
+void launch_form(const BmmPlan& p, uint32_t grid, hipStream_t stream) {
+  if constexpr (SHORT)
+    hipLaunchKernelGGL((bmm_short_kernel<W, PR, QR>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else
+    hipLaunchKernelGGL((bmm_kernel<bmm_depth(W), W, PR, QR>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+}
+
+template <bool SHORT, int W>
+void launch_bmm(const BmmPlan& p, bool pr, bool qr, uint32_t grid, hipStream_t stream) {
+  if (pr && qr) launch_form<SHORT, W, true, true>(p, grid, stream);
+  else if (pr) launch_form<SHORT, W, true, false>(p, grid, stream);
+  else if (qr) launch_form<SHORT, W, false, true>(p, grid, stream);
+  else launch_form<SHORT, W, false, false>(p, grid, stream);
 }
 
 // ---------------------------------------------------------------- host
 
-// b's columns run contiguously along k in 16-byte aligned groups of 8: unit
-// step along k (a plain axis of stride 1, or a blocked axis of in-block stride
-// 1 whose block is a multiple of 8 and whose block stride keeps 8-alignment),
-// 8-aligned column, batch and group offsets, a 16-byte aligned base.
-bool streamable_b(const Mat& b) {
-  const Axis& k = b.row;
-  const bool unit = (k.blk.d == 1 && k.outer == 1) || (k.blk.d % 8 == 0 && k.inner == 1 && k.outer % 8 == 0);
-  const bool cols = b.col.outer % 8 == 0 && (b.col.blk.d == 1 || b.col.inner % 8 == 0);
-  return unit && cols && reinterpret_cast<uintptr_t>(b.p) % 16 == 0 && b.batch % 8 == 0 && b.row_origin % 8 == 0 &&
-         b.row_group % 8 == 0;
+// Runs of `n` consecutive indexes from multiples of n are adjacent in memory:
+// a plain axis of stride 1, or a blocked axis of in-block stride 1 whose
+// blocks, origin and per-batch origin hold whole runs.
+bool runs_of(const Axis& x, uint32_t origin, uint32_t group, uint32_t n) {
+  if (x.blk.d == 1) return x.outer == 1;
+  return x.inner == 1 && x.blk.d % n == 0 && origin % n == 0 && group % n == 0;
 }
 
 // Rows and columns of an operand before transposition (bmm_flow.cpp:280-281).
@@ -576,90 +800,117 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
                      x->sizes[2] < ((int64_t)1 << 31),
                  THIN_ERR_UNSUPPORTED, "bmm: operand dimensions exceed the kernel index range");
 
+  const Mat am = make_input(a, layout->transpose_a, layout->groups, layout->a_offset);
+  const Mat bm = make_input(b, layout->transpose_b, layout->groups, layout->b_offset);
+  // k is the column axis of a and the row axis of b
+  Side sa, sb;
+  memset(&sa, 0, sizeof sa);
+  memset(&sb, 0, sizeof sb);
+  sa.p = am.p;
+  sa.batch = am.batch;
+  sa.row = am.row;
+  sa.step = am.col;
+  sa.row_origin = am.row_origin;
+  sa.row_group = am.row_group;
+  sa.step_origin = am.col_origin;
+  sa.step_group = am.col_group;
+  sa.rows = (uint32_t)s.m;
+  sb.p = bm.p;
+  sb.batch = bm.batch;
+  sb.row = bm.col;
+  sb.step = bm.row;
+  sb.row_origin = bm.col_origin;
+  sb.row_group = bm.col_group;
+  sb.step_origin = bm.row_origin;
+  sb.step_group = bm.row_group;
+  sb.rows = (uint32_t)s.n;
+
   BmmPlan p;
   memset(&p, 0, sizeof p);
-  p.a = make_input(a, layout->transpose_a, layout->groups, layout->a_offset);
-  p.b = make_input(b, layout->transpose_b, layout->groups, layout->b_offset);
-  Mat& y = p.y;
-  y.p = static_cast<_Float16*>(out->data);
+  p.y = static_cast<_Float16*>(out->data);
+  p.k = (uint32_t)s.k;
+  const Axis cols = make_axis(1, out->strides[2], 0);
   if (!layout->blocked_output) {
-    y.batch = out->strides[0];
-    y.row = make_axis(1, out->strides[1], 0);
-    y.col = make_axis(1, out->strides[2], 0);
+    // rows of n outputs: p is b's columns
+    p.P = sb;
+    p.Q = sa;
+    p.ybatch = out->strides[0];
+    p.yp = cols;
+    p.yq = make_axis(1, out->strides[1], 0);
   } else {
     // channel r of batch b is packed channel b * m + r of [lead, C1, n, 16]
     // (grouped), or channel r of image b (ungrouped; the two agree when the
-    // ungrouped tensor is contiguous)
-    y.row = make_axis(16, out->strides[1], out->strides[3]);
-    y.col = make_axis(1, out->strides[2], 0);
-    if (layout->groups) {
-      y.batch = 0;
-      y.row_group = (uint32_t)s.m;
-    } else {
-      y.batch = out->strides[0];
-    }
+    // ungrouped tensor is contiguous); p is the channels
+    p.P = sa;
+    p.Q = sb;
+    p.yp = make_axis(16, out->strides[1], out->strides[3]);
+    p.yq = cols;
+    if (layout->groups) p.yp_group = (uint32_t)s.m;
+    else p.ybatch = out->strides[0];
   }
-  p.m = (uint32_t)s.m;
-  p.n = (uint32_t)s.n;
-  p.k = (uint32_t)s.k;
-  // k is the column axis of a and the row axis of b
-  p.a_kfast = unit_step(p.a.col) <= unit_step(p.a.row);
-  p.b_kfast = unit_step(p.b.row) <= unit_step(p.b.col);
-  p.ntiles = (uint32_t)((s.n + kBmmCols - 1) / kBmmCols);
-  int64_t b_extent = 1;  // elements from b's data pointer to its last element, + 1
-  for (int d = 0; d < b->rank; ++d) b_extent += (b->sizes[d] - 1) * b->strides[d];
-  if (streamable_b(p.b) && b_extent * 2 < ((int64_t)1 << 31)) {
-    p.b_bytes = (uint32_t)(b_extent * 2);
-    p.b_vrun = p.b.row.blk.d == 1 ? 0u : p.b.row.blk.d / 8u;
-    p.b_vjump = p.b.row.blk.d == 1 ? 0u : (uint32_t)((p.b.row.outer - p.b.row.blk.d) * 2);
-    if (p.k % 8 == 0 && p.b.col.blk.d == 1 && p.b.col.outer >= 64) {
-      // columns a line or more apart: 64-column tiles staged through LDS
-      auto blocks = [&](int rm) { return (uint64_t)s.batch * ((s.m + 4 * rm - 1) / (4 * rm)) * p.ntiles; };
-      const int rm = blocks(4) * 4 >= 1024 ? 4 : blocks(2) * 4 >= 1024 ? 2 : 1;
-      p.mtiles = (uint32_t)((s.m + 4 * rm - 1) / (4 * rm));
-      const uint64_t grid = blocks(rm);
-      THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
-      if (rm == 4)
-        hipLaunchKernelGGL(bmm_tile_kernel<4>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-      else if (rm == 2)
-        hipLaunchKernelGGL(bmm_tile_kernel<2>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-      else
-        hipLaunchKernelGGL(bmm_tile_kernel<1>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-      THIN_LAUNCH_CHECK("bmm_tile_kernel");
-      return THIN_OK;
-    }
-    // rows per wave: 2, which measured fastest for both attention products
-    // (q^T k [4,400,32]x[4,32,400]: 6.3 us rotated against 6.9 with 4 rows and
-    // 7.7 with 1); 1 when that leaves under half a wave per SIMD, 4 when it
-    // would queue more than 8 waves per SIMD
-    auto waves = [&](int rm) { return (uint64_t)s.batch * ((s.m + rm - 1) / rm) * p.ntiles; };
-    const int rm = waves(2) < 512 ? 1 : waves(2) > 8192 ? 4 : 2;
-    p.mtiles = (uint32_t)((s.m + rm - 1) / rm);
-    p.div_mt = FastDiv::make(p.mtiles);
-    p.div_nt = FastDiv::make(p.ntiles);
-    const uint64_t grid = waves(rm);
-    THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
-    if (rm == 4)
-      launch_stream<4>(p, (uint32_t)grid, stream);
-    else if (rm == 2)
-      launch_stream<2>(p, (uint32_t)grid, stream);
-    else
-      launch_stream<1>(p, (uint32_t)grid, stream);
-    THIN_LAUNCH_CHECK("bmm_stream_kernel");
-    return THIN_OK;
+  // 64 x 64 blocks (four matrix products per operand pair read) where they
+  // give every compute unit two, else 32 x 32 ones, which spread the work
+  // over four times as many waves
+  auto blocks = [&](uint64_t r) { return (uint64_t)s.batch * ((p.P.rows + r - 1) / r) * ((p.Q.rows + r - 1) / r); };
+  uint32_t w = blocks(64) >= 512 ? 2 : 1;
+  // whole 16-byte runs along the steps, else along the rows (rows of a plain
+  // axis may end in a partial run: the last tile then starts early, which
+  // takes a tile before it); the kernels' lane offsets are 32-bit
+  auto steps_runs = [&](const Side& x) { return s.k >= 8 && runs_of(x.step, x.step_origin, x.step_group, 8); };
+  auto rows_runs = [&](const Side& x) {
+    return runs_of(x.row, x.row_origin, x.row_group, 8) &&
+           (x.rows % 8 == 0 || (x.row.blk.d == 1 && x.rows > 32u * w));
+  };
+  auto near = [](const thin_desc* d) {
+    int64_t extent = 0;
+    for (int i = 1; i < d->rank; ++i) extent += (d->sizes[i] - 1) * d->strides[i];
+    return extent < ((int64_t)1 << 30);
+  };
+  const bool fast = (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)) && near(a) && near(b) &&
+                    32 % p.P.row.blk.d == 0 && 32 % p.P.step.blk.d == 0 && 32 % p.Q.step.blk.d == 0;
+  if (!fast) w = 1;
+  const bool one = s.k <= 32;  // one chunk of steps
+  const uint32_t r = 32 * w, kd = (uint32_t)bmm_depth((int)w);
+  const bool pr = !steps_runs(p.P), qr = !steps_runs(p.Q);
+  p.P.steps_near = unit_step(p.P.step) <= unit_step(p.P.row);
+  p.Q.steps_near = unit_step(p.Q.step) <= unit_step(p.Q.row);
+  const uint32_t rp = fast ? r : p.Q.rows <= 16 ? 64 : p.P.rows <= 16 ? 16 : 32, rq = fast ? r : 1024 / rp;
+  p.ptiles = (p.P.rows + rp - 1) / rp;
+  p.qtiles = FastDiv::make((p.Q.rows + rq - 1) / rq);
+  p.y_vec = runs_of(p.yp, 0, p.yp_group, 4 * w) ? 1u : 0u;
+  THIN_REQUIRE(blocks(r) < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
+  p.span = 1;
+  if (fast && one) {
+    // as many P tiles a block as leave about three blocks a compute unit, in
+    // even shares (q^T k: [128,400,32] x [128,32,400] 26.1 us with one tile a
+    // block and 24.3 with all seven, [4,1600,32] x [4,32,1600] 13.7 us with up
+    // to four and 16.0 with seven)
+    const uint64_t share = blocks(r) / 800;
+    const uint32_t most = share < 1 ? 1u : share > 8 ? 8u : (uint32_t)share;
+    const uint32_t parts = (p.ptiles + most - 1) / most;
+    p.span = (p.ptiles + parts - 1) / parts;
+    p.P.hop = (int64_t)(r / p.P.row.blk.d) * p.P.row.outer * 2;
+    p.yhop = (int64_t)(r / p.yp.blk.d) * p.yp.outer;
+  } else if (fast) {
+    p.P.hop = (int64_t)(kd / p.P.step.blk.d) * p.P.step.outer * 2;
+    p.Q.hop = (int64_t)(kd / p.Q.step.blk.d) * p.Q.step.outer * 2;
   }
-  // rows per wave: the widest tile that still gives every SIMD about one wave
-  auto blocks = [&](int rm) { return (uint64_t)s.batch * ((s.m + 4 * rm - 1) / (4 * rm)) * p.ntiles; };
-  const int rm = blocks(4) * 4 >= 1024 ? 4 : blocks(2) * 4 >= 1024 ? 2 : 1;
-  p.mtiles = (uint32_t)((s.m + 4 * rm - 1) / (4 * rm));
-  const uint64_t grid = blocks(rm);
-  THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
-  if (rm == 4)
-    hipLaunchKernelGGL(bmm_kernel<4>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-  else if (rm == 2)
-    hipLaunchKernelGGL(bmm_kernel<2>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
+  p.pblocks = FastDiv::make((p.ptiles + p.span - 1) / p.span);
+  const uint32_t grid = (uint32_t)((uint64_t)s.batch * p.qtiles.d * p.pblocks.d);
+  if (!fast && rp == 64)
+    hipLaunchKernelGGL((bmm_gather_kernel<64, 16>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else if (!fast && rp == 16)
+    hipLaunchKernelGGL((bmm_gather_kernel<16, 64>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else if (!fast)
+    hipLaunchKernelGGL((bmm_gather_kernel<32, 32>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else if (one && w == 2)
+    launch_bmm<true, 2>(p, pr, qr, grid, stream);
+  else if (one)
+    launch_bmm<true, 1>(p, pr, qr, grid, stream);
+  else if (w == 2)
+    launch_bmm<false, 2>(p, pr, qr, grid, stream);
   else
-    hipLaunchKernelGGL(bmm_kernel<1>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
+    launch_bmm<false, 1>(p, pr, qr, grid, stream);
   THIN_LAUNCH_CHECK("bmm_kernel");
   return THIN_OK;
 }
