@@ -184,3 +184,51 @@ def test_selection_graph_replays(gpu, noalloc):
         # eager calls between replays
         for dv, k, eager in cases:
             assert bits_equal(capi.detection_select(dv, k, noalloc=noalloc).cpu(), eager.cpu())
+
+
+def _scores_case(kind, batch, anchors, nc, seed):
+    """Independent scores; all the best ones within a few hundred neighbouring
+    anchors (more candidates in a run than are held of a long image); or eight
+    score levels (thousands of ties)."""
+    g = torch.Generator().manual_seed(seed)
+    s = torch.rand(batch, anchors, nc, generator=g)
+    if kind == "clustered":
+        first = anchors // 3
+        s = s * 0.25
+        s[:, first:first + 450] += 0.5
+    elif kind == "tied":
+        s = (s * 8).floor() / 8
+    boxes = torch.randn(batch, anchors, 4, generator=g)
+    return torch.cat((boxes, s), -1).half()
+
+
+@pytest.mark.parametrize("kind", ["independent", "clustered", "tied"])
+@pytest.mark.parametrize("batch,anchors,nc,max_det,layout", [
+    (1, 16385, 6, 300, "transposed"),   # first size past the runs held whole, scalar loads
+    (2, 33600, 8, 300, "transposed"),   # 1280 x 1280 pixels; 526 runs: 128 threads each
+    (1, 33600, 8, 300, "contiguous"),
+    (1, 65536, 5, 1024, "transposed"),  # the most anchors and records
+    (1, 65537, 5, 300, "transposed"),   # one more: the one-workgroup path
+    (9, 8400, 12, 300, "transposed"),   # many runs of images held whole
+    (4, 16384, 7, 1000, "transposed"),
+    (1, 130, 4, 130, "transposed"),     # K the whole image: no rank bounds it
+    (2, 1000, 4, 1000, "contiguous"),   # K close to the anchors
+    (3, 300, 4, 200, "transposed"),
+])
+def test_selection_run_bounds(gpu, kind, batch, anchors, nc, max_det, layout):
+    x = _scores_case(kind, batch, anchors, nc, anchors + nc)
+    run_case(gpu, x, max_det, False, layout, f"{kind}-{batch}x{anchors}x{nc}-{max_det}")
+
+
+def test_selection_scratch_sizes(gpu):
+    """Calls whose two-launch workspace is larger than the static scratch, or
+    than the workspace given, still run where the other paths' fits."""
+    from thintnpu_amd import capi
+    x = _scores_case("independent", 12, 33600, 5, 3)
+    expect = sel.select(x, 300, False)["output"]
+    assert capi.detection_select_workspace(12, 33600, 5, 300, False) > capi.SELECT_SCRATCH_BYTES
+    d = x.to(gpu)
+    assert bits_equal(capi.detection_select(d, 300, noalloc=True).cpu(), expect)
+    small = torch.empty(4 << 20, dtype=torch.uint8, device=gpu)
+    assert bits_equal(capi.detection_select(d, 300, workspace=small).cpu(), expect)
+    assert bits_equal(capi.detection_select(d, 300).cpu(), expect)

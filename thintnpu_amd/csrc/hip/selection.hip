@@ -20,6 +20,8 @@
 
 #include <string.h>
 
+#include <math.h>
+
 #include <algorithm>
 #include <mutex>
 
@@ -1275,10 +1277,10 @@ __global__ __launch_bounds__(kSplitThreads) void merge2_kernel(SplitPlan p) {
 // records are sorted.  Records are unique, so the network's order is the
 // stable (key, index) order.
 constexpr uint32_t kRun = 128;             // anchors per sorted run
-constexpr uint32_t kRunThreads = 512;      // runs_kernel workgroups
-constexpr uint32_t kMaxRuns = 128;         // runs per image (A <= 16384)
-constexpr uint32_t kRunPitch = kRun + 4;   // finish LDS words per run list (run l on banks 4l mod 64)
-constexpr uint32_t kSidePitch = kRun + 8;  // finish LDS halves per run row-key list (16-byte rows)
+constexpr uint32_t kRunThreads = 512;      // runs_kernel workgroups of a few images
+constexpr uint32_t kRunManyThreads = 128;  // and of many runs
+constexpr uint32_t kHeldRuns = 128;        // runs per image that finish_kernel holds whole
+constexpr uint32_t kMaxRuns = 512;         // runs per image (A <= 65536)
 constexpr uint32_t kFinishThreads = 1024;  // finish_kernel workgroups
 constexpr uint32_t kSortCap = 1024;        // records one bitonic sort holds
 constexpr uint32_t kPairTable = 32768;     // K * nc limit: every stage-1 row in LDS (fallback)
@@ -1287,22 +1289,20 @@ constexpr uint32_t kMaxX = 256;            // prefetched candidate rows
 constexpr uint32_t kXTable = 16384;        // their fp16 scores in LDS
 constexpr uint32_t kXBatch = 8;            // prefetched row loads per thread
 constexpr uint32_t kNoX = 0xffffu;
-// finish_kernel's reused LDS region (32-bit words): the runs and their side
-// keys, then the candidate tables, then (fallback) the pair table; info1
-// lies past the pair table and survives it.
-constexpr uint32_t kRegSide = kMaxRuns * kRunPitch;            // runs: row keys (u16)
-constexpr uint32_t kRegWords = kRegSide + kMaxRuns * kSidePitch / 2;
+// finish_kernel's reused LDS region (32-bit words): the candidate tables,
+// then (fallback) the pair table; info1 lies past the pair table and survives
+// it.
 constexpr uint32_t kRegInfoSlot = 8192;                        // u4v [kSortCap]: info per slot
 constexpr uint32_t kRegXTable = kRegInfoSlot + 4 * kSortCap;   // u16 [kXTable]
 constexpr uint32_t kRegInfo1 = kRegXTable + kXTable / 2;       // u4v [kSplitMaxK]: info per stage-1 rank
-static_assert(kRegInfo1 + 4 * kSplitMaxK <= kRegWords, "finish LDS region");
-static_assert(kPairTable / 2 <= kRegInfo1 && kMaxRuns * kRun / 2 <= kRegInfoSlot, "finish LDS aliasing");
+constexpr uint32_t kRegWords = kRegInfo1 + 4 * kSplitMaxK;
+static_assert(kPairTable / 2 <= kRegInfo1, "finish LDS aliasing");
 
 struct RunsPlan {
   Layout L;
   uint32_t A, nc, K;
   uint32_t runs;          // runs per image: ceil(A / kRun)
-  uint32_t q;             // prefix length whose run prefixes hold K records (host: A and K only)
+  uint32_t q, m, m2;      // finish: prefix length and ranks of the candidate bounds (host: A and K only)
   uint32_t rows_per;      // finish: stage-1 ranks per gather pass, kFinishThreads / nc
   int32_t agnostic;
   int32_t vec_classes;    // anchors contiguous in aligned 16-byte groups
@@ -1557,55 +1557,70 @@ __device__ __forceinline__ uint32_t run_key2(uint32_t w) {
   return key & __builtin_bit_cast(uint32_t, t >> (i16x2)15);
 }
 
-// Folds (key << 16 | class) k of a later class, score bits h, into the three
-// smallest so far (b < s < t; kPad where missing): every key is distinct, so
-// the new third is the middle of (s, k, t) and the new second the middle of
-// (b, k, s).
-__device__ __forceinline__ void fold3(uint32_t& b, uint32_t& s, uint32_t& t, uint32_t& bits, uint32_t k, uint32_t h) {
+// Folds (key << 16 | class) k into the three smallest so far (b < s < t;
+// kPad where missing): every key is distinct, so the new third is the middle
+// of (s, k, t) and the new second the middle of (b, k, s).
+__device__ __forceinline__ void fold3(uint32_t& b, uint32_t& s, uint32_t& t, uint32_t k) {
   t = umed3(s, k, t);
   s = umed3(b, k, s);
-  if (k < b) {
-    b = k;
-    bits = h;
-  }
+  b = min(b, k);
+}
+// The folds of an anchor's three into another's.
+__device__ __forceinline__ void fold_three(uint32_t& b, uint32_t& s, uint32_t& t, uint32_t pb, uint32_t ps, uint32_t pt) {
+  fold3(b, s, t, pb);
+  fold3(b, s, t, ps);
+  fold3(b, s, t, pt);
+}
+// Two anchors' scores of class c, the halves of w.  PLAIN: neither is negative
+// or NaN, so that 0x7fff - |h| is the key, one xor for both.
+template <bool PLAIN>
+__device__ __forceinline__ void fold_word(uint32_t w, uint32_t c, uint32_t& b0, uint32_t& s0, uint32_t& t0,
+                                          uint32_t& b1, uint32_t& s1, uint32_t& t1) {
+  const uint32_t kw = PLAIN ? w ^ 0x7fff7fffu : run_key2(w);
+  fold3(b0, s0, t0, (kw << 16) | c);
+  fold3(b1, s1, t1, (kw & 0xffff0000u) | c);
 }
 
 // Class keys of kRun anchors (the two load forms of slice_kernel, and a row
 // form for rows of contiguous classes) and their box channels; then the
 // run's records sorted: waves 0 and 1 sort 64 each (ascending, descending),
 // one LDS exchange at distance 64 and the in-wave end of the last merge.
+//
+// kRunManyThreads: the octet form alone, eight class groups in 15 KB of LDS
+// instead of 32 in 66 KB, for launches of many runs: ten groups of waves fit a
+// compute unit where two did, and a run merges a quarter of the triples.
+template <uint32_t kRunThreads>
 __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
+  constexpr bool kMany = kRunThreads == kRunManyThreads;
   constexpr uint32_t kTiles = kRun / 64;                  // scalar form: 64-anchor tiles
   constexpr uint32_t kGroups = kRunThreads / kRun;        // scalar form: class groups per anchor
   constexpr uint32_t kUnroll = 16;                        // scalar form: class loads in flight per lane
   constexpr uint32_t kOctets = kRun / 8;
   constexpr uint32_t kVGroups = kRunThreads / kOctets;    // vector form: class groups per octet
-  constexpr uint32_t kVUnroll = 4;                        // vector form: 16-byte loads in flight per lane
+  constexpr uint32_t kVUnroll = kMany ? 5 : 4;            // vector form: 16-byte loads in flight per lane
   constexpr uint32_t kRUnroll = 6;                        // row form: 8-byte loads in flight per lane
-  static_assert(kRunThreads == 4 * kRun, "row form: four lanes per anchor");
+  static_assert(kMany || kRunThreads == 4 * kRun, "row form: four lanes per anchor");
   constexpr uint32_t kParts = kRunThreads / kRun;         // group-reduction parts per anchor
-  static_assert(kVGroups == kParts * 8 && kGroups == kParts && kGroups == 4, "group reduction shape");
-  // per class group and anchor: the three smallest (key << 16 | class), best bits
+  static_assert(kVGroups == kParts * 8 && kGroups == kParts && (kMany || kGroups == 4), "group reduction shape");
+  // per class group and anchor: the three smallest (key << 16 | class)
   __shared__ uint32_t g_b[kVGroups * kRun], g_s[kVGroups * kRun], g_t[kVGroups * kRun];
-  __shared__ uint16_t g_bits[kVGroups * kRun];
-  __shared__ uint32_t part_b[kParts * kRun], part_s[kParts * kRun], part_t[kParts * kRun];
-  __shared__ uint16_t part_bits[kParts * kRun];
+  constexpr uint32_t kPart = kMany ? 1 : kParts * kRun;
+  __shared__ uint32_t part_b[kPart], part_s[kPart], part_t[kPart];
   __shared__ uint16_t box[4 * kRun];
   __shared__ uint16_t side_of[kRun];
   __shared__ uint32_t xch[kRun];
   const uint32_t b = blockIdx.y, run = blockIdx.x, tid = threadIdx.x;
   const uint16_t* img = p.L.x + b * p.L.sb;
   const uint32_t sc = (uint32_t)p.L.sc;
-  if (p.vec_classes) {
+  if (kMany || p.vec_classes) {
     const uint32_t o = tid % kOctets, g = tid / kOctets;
     const uint32_t a0 = run * kRun + o * 8u;
-    uint32_t kb[8], ks[8], kt[8], bits[8];
+    uint32_t kb[8], ks[8], kt[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       kb[j] = kPad;
       ks[j] = kPad;
       kt[j] = kPad;
-      bits[j] = 0;
     }
     if (a0 < p.A) {  // A % 8 == 0: the octet is whole
       // box channel g of the octet (groups 0-3), in flight with the classes
@@ -1617,18 +1632,30 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
           const uint32_t c = c0 + u * kVGroups;
           v[u] = c < p.nc ? *reinterpret_cast<const u4v*>(img + (4u + c) * sc + a0) : (u4v)0u;
         }
+        // sigmoid scores are all plain; a wave with any other takes the full keys
+        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 most = (u16x2)0;
 #pragma unroll
-        for (uint32_t u = 0; u < kVUnroll; ++u) {
-          const uint32_t c = c0 + u * kVGroups;
-          if (c < p.nc) {
+        for (uint32_t u = 0; u < kVUnroll; ++u)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {  // two anchors per 32-bit word
-              const uint32_t w = v[u][q], kw = run_key2(w);
-              fold3(kb[2 * q], ks[2 * q], kt[2 * q], bits[2 * q], (kw << 16) | c, w & 0xffffu);
-              fold3(kb[2 * q + 1], ks[2 * q + 1], kt[2 * q + 1], bits[2 * q + 1], (kw & 0xffff0000u) | c, w >> 16);
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t w = v[u][q];
+            most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, w));
+          }
+        auto fold = [&](auto plain) __attribute__((always_inline)) {
+#pragma unroll
+          for (uint32_t u = 0; u < kVUnroll; ++u) {
+            const uint32_t c = c0 + u * kVGroups;
+            if (c < p.nc) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q)  // two anchors per 32-bit word
+                fold_word<decltype(plain)::value>(v[u][q], c, kb[2 * q], ks[2 * q], kt[2 * q], kb[2 * q + 1],
+                                                  ks[2 * q + 1], kt[2 * q + 1]);
             }
           }
-        }
+        };
+        if (__any(most[0] > 0x7c00u || most[1] > 0x7c00u)) fold(std::false_type());
+        else fold(std::true_type());
       }
       if (g < 4) {
 #pragma unroll
@@ -1641,15 +1668,15 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
       g_b[at] = kb[j];
       g_s[at] = ks[j];
       g_t[at] = kt[j];
-      g_bits[at] = (uint16_t)bits[j];
     }
+  } else if constexpr (kMany) {
   } else if (p.row_classes) {
     // four lanes per anchor: lane g reads the anchor's 8-byte class chunks g,
     // g + 4, ... (lane 0 also the box chunk before them), then the quad merges
     // its four triples in two exchanges, leaving the anchor's three in every lane
     typedef uint32_t u2v __attribute__((ext_vector_type(2)));
     const uint32_t local = tid / 4u, g = tid % 4u, a = run * kRun + local, nch = p.nc / 4u;
-    uint32_t kb = kPad, ks = kPad, kt = kPad, bb = 0u;
+    uint32_t kb = kPad, ks = kPad, kt = kPad;
     u2v bx = (u2v)0u;
     if (a < p.A) {
       // one image spans fewer than 2^31 elements (checked on the host)
@@ -1669,28 +1696,19 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
 #pragma unroll
             for (uint32_t q = 0; q < 2; ++q) {  // classes 4j + 2q and 4j + 2q + 1
               const uint32_t w = v[u][q], kw = run_key2(w), c = 4u * j + 2u * q;
-              fold3(kb, ks, kt, bb, (kw << 16) | c, w & 0xffffu);
-              fold3(kb, ks, kt, bb, (kw & 0xffff0000u) | (c + 1u), w >> 16);
+              fold3(kb, ks, kt, (kw << 16) | c);
+              fold3(kb, ks, kt, (kw & 0xffff0000u) | (c + 1u));
             }
           }
         }
       }
     }
-    auto merge = [&](uint32_t pb, uint32_t ps, uint32_t pt, uint32_t ph) {
-      uint32_t unused = 0;
-      fold3(kb, ks, kt, bb, pb, ph);
-      fold3(kb, ks, kt, unused, ps, 0u);  // never below the partner's best, so bits stay
-      fold3(kb, ks, kt, unused, pt, 0u);
-    };
-    merge(dev::lane_xor_bits<1>(kb), dev::lane_xor_bits<1>(ks), dev::lane_xor_bits<1>(kt),
-          dev::lane_xor_bits<1>(bb));
-    merge(dev::lane_xor_bits<2>(kb), dev::lane_xor_bits<2>(ks), dev::lane_xor_bits<2>(kt),
-          dev::lane_xor_bits<2>(bb));
+    fold_three(kb, ks, kt, dev::lane_xor_bits<1>(kb), dev::lane_xor_bits<1>(ks), dev::lane_xor_bits<1>(kt));
+    fold_three(kb, ks, kt, dev::lane_xor_bits<2>(kb), dev::lane_xor_bits<2>(ks), dev::lane_xor_bits<2>(kt));
     if (g == 0) {
       g_b[local] = kb;
       g_s[local] = ks;
       g_t[local] = kt;
-      g_bits[local] = (uint16_t)bb;
 #pragma unroll
       for (uint32_t c = 0; c < 4; ++c) box[c * kRun + local] = (uint16_t)(bx[c / 2] >> (16 * (c & 1)));
     }
@@ -1698,7 +1716,7 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t local = (wave % kTiles) * 64u + lane, grp = wave / kTiles;
     const uint32_t a = run * kRun + local;
-    uint32_t kb = kPad, ks = kPad, kt = kPad, bb = 0u;
+    uint32_t kb = kPad, ks = kPad, kt = kPad;
     if (a < p.A) {
       // one image spans fewer than 2^31 elements (checked on the host)
       const uint32_t base = a * (uint32_t)p.L.sa;
@@ -1714,7 +1732,7 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
 #pragma unroll
         for (uint32_t u = 0; u < kUnroll; ++u) {
           const uint32_t c = c0 + u * kGroups;
-          if (c < p.nc) fold3(kb, ks, kt, bb, (run_key(bits[u]) << 16) | c, bits[u]);
+          if (c < p.nc) fold3(kb, ks, kt, (run_key(bits[u]) << 16) | c);
         }
       }
       box[grp * kRun + local] = (uint16_t)bxv;
@@ -1723,64 +1741,57 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
     g_b[at] = kb;
     g_s[at] = ks;
     g_t[at] = kt;
-    g_bits[at] = (uint16_t)bb;
   }
   __syncthreads();
   // The three smallest over the class groups of each anchor (all keys
   // distinct, so any merge order gives the same three); the vector form's 32
   // groups reduce in two levels.
-  auto reduce = [&](const uint32_t* bs, const uint32_t* ss, const uint32_t* ts, const uint16_t* hs, auto count,
-                    uint32_t first, uint32_t& kb, uint32_t& ks, uint32_t& kt, uint32_t& bb) {
+  auto reduce = [&](const uint32_t* bs, const uint32_t* ss, const uint32_t* ts, auto count, uint32_t first, uint32_t& kb,
+                    uint32_t& ks, uint32_t& kt) {
     constexpr uint32_t N = decltype(count)::value;
-    uint32_t vb[N], vs[N], vt[N], vh[N];
+    uint32_t vb[N], vs[N], vt[N];
 #pragma unroll
     for (uint32_t g = 0; g < N; ++g) {
       const uint32_t at = (first + g) * kRun;
       vb[g] = bs[at];
       vs[g] = ss[at];
       vt[g] = ts[at];
-      vh[g] = hs[at];
     }
     kb = vb[0];
     ks = vs[0];
     kt = vt[0];
-    bb = vh[0];
 #pragma unroll
-    for (uint32_t g = 1; g < N; ++g) {
-      fold3(kb, ks, kt, bb, vb[g], vh[g]);
-      uint32_t unused = 0;
-      fold3(kb, ks, kt, unused, vs[g], 0u);  // never below the group's best, so bits stay
-      fold3(kb, ks, kt, unused, vt[g], 0u);
-    }
+    for (uint32_t g = 1; g < N; ++g) fold_three(kb, ks, kt, vb[g], vs[g], vt[g]);
   };
-  uint32_t kb = kPad, ks = kPad, kt = kPad, bb = 0u;
-  if (p.vec_classes) {
+  uint32_t kb = kPad, ks = kPad, kt = kPad;
+  if constexpr (kMany) {
+    reduce(g_b + tid, g_s + tid, g_t + tid, std::integral_constant<uint32_t, 8>(), 0u, kb, ks, kt);
+  } else if (p.vec_classes) {
     const uint32_t x = tid % kRun, q = tid / kRun;
-    reduce(g_b + x, g_s + x, g_t + x, g_bits + x, std::integral_constant<uint32_t, 8>(), q * 8u, kb, ks, kt, bb);
+    reduce(g_b + x, g_s + x, g_t + x, std::integral_constant<uint32_t, 8>(), q * 8u, kb, ks, kt);
     part_b[q * kRun + x] = kb;
     part_s[q * kRun + x] = ks;
     part_t[q * kRun + x] = kt;
-    part_bits[q * kRun + x] = (uint16_t)bb;
     __syncthreads();
     if (tid < kRun)
-      reduce(part_b + tid, part_s + tid, part_t + tid, part_bits + tid, std::integral_constant<uint32_t, kParts>(), 0u,
-             kb, ks, kt, bb);
+      reduce(part_b + tid, part_s + tid, part_t + tid, std::integral_constant<uint32_t, kParts>(), 0u, kb, ks, kt);
   } else if (p.row_classes) {
     if (tid < kRun) {
       kb = g_b[tid];
       ks = g_s[tid];
       kt = g_t[tid];
-      bb = g_bits[tid];
     }
   } else if (tid < kRun) {
-    reduce(g_b + tid, g_s + tid, g_t + tid, g_bits + tid, std::integral_constant<uint32_t, kGroups>(), 0u, kb, ks, kt,
-           bb);
+    reduce(g_b + tid, g_s + tid, g_t + tid, std::integral_constant<uint32_t, kGroups>(), 0u, kb, ks, kt);
   }
   uint32_t rec = kPad;
   if (tid < kRun) {
     const uint32_t a = run * kRun + tid;
     if (a < p.A) {
       const size_t t = (size_t)b * p.A + a;
+      // the class-max score's bits: of its key, or (NaN, zero) as stored
+      const uint32_t key = kb >> 16;
+      const uint32_t bb = key_ambiguous(key) ? img[a * (uint32_t)p.L.sa + (4u + (kb & 0xffffu)) * sc] : key_bits(key);
       u4v iv;
       iv[0] = box[tid] | ((uint32_t)box[kRun + tid] << 16);
       iv[1] = box[2 * kRun + tid] | ((uint32_t)box[3 * kRun + tid] << 16);
@@ -1807,118 +1818,161 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
 }
 
 // Stage-1 candidates, their sort, stage 2 and the rows, for image blockIdx.x.
+//
+// Eight threads hold a run, in registers: all of it where the image has at
+// most kHeldRuns runs, otherwise (WIDE) its first 32 records, four runs to
+// the eight threads, and a run that has more candidates than that is read on
+// from memory.
+//
+// Candidates are the records up to a bound R that at least K records meet.
+// The q-th records of the runs, ordered: the m-th one has m runs with q
+// records up to it, so with m * q >= K it is such a bound; the m2-th is lower
+// and meets K records too for most inputs (the host takes the rank where
+// independent scores would leave about 1.25 K), so it is the bound when the
+// count says so.  Taking the largest of the q-th records instead, as this
+// kernel did, left 760 candidates of 8400 anchors for K = 300 on average and
+// over 1024 for one image in thirty, which then took the radix select and
+// the full gather: 44 us for a batch of 32 images, 10 for one image.
+template <bool WIDE>
 __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   __shared__ __attribute__((aligned(16))) uint32_t region[kRegWords];
   __shared__ uint32_t sortbuf[kSortCap], s2buf[kSortCap + 64];  // s2buf: K pairs and up to 64 extras
   __shared__ uint32_t xch[2 * kSortCap];
   __shared__ uint16_t anchor_of[kSortCap], xslot[kSortCap], xlist[kMaxX], xrank[kSortCap], anchors1[kSplitMaxK],
       x1[kSplitMaxK];
-  __shared__ uint32_t cnt[kMaxRuns], off[kMaxRuns + 1];
-  __shared__ uint32_t hist[256], sel[2], bound, count, count2, nx, nxr;
+  constexpr uint32_t kRuns = WIDE ? kMaxRuns : kHeldRuns;
+  __shared__ __attribute__((aligned(16))) uint32_t qth[kRuns];
+  __shared__ uint32_t cnt[kRuns], cnt2[kRuns], off[kRuns];
+  __shared__ uint32_t hist[256], sel[2], bound[2], chosen, total, count, count2, nx, nxr;
   const uint32_t b = blockIdx.x, tid = threadIdx.x, nl = p.runs, K = p.K, nc = p.nc;
   const uint16_t* img = p.L.x + b * p.L.sb;
   const uint32_t sa = (uint32_t)p.L.sa, sc = (uint32_t)p.L.sc;
-  uint32_t* lists = region;
-  uint16_t* lside = reinterpret_cast<uint16_t*>(region + kRegSide);
   u4v* info_slot = reinterpret_cast<u4v*>(region + kRegInfoSlot);
   uint16_t* xtable = reinterpret_cast<uint16_t*>(region + kRegXTable);
   u4v* info1 = reinterpret_cast<u4v*>(region + kRegInfo1);
   uint16_t* table = reinterpret_cast<uint16_t*>(region);  // fallback: [K * nc]
   const u4v* info_g = p.info + (size_t)b * p.A;
 
-  // the runs and their row keys into LDS: every 16-byte load issued before
-  // any is stored
-  {
-    constexpr uint32_t kV = kRun / 4, kPer = kMaxRuns * kV / kFinishThreads;
-    constexpr uint32_t kSV = kRun / 8, kSPer = kMaxRuns * kSV / kFinishThreads;
-    const uint32_t total = nl * kV, stotal = nl * kSV;
-    const u4v* src = reinterpret_cast<const u4v*>(p.runs_rec + (size_t)b * nl * kRun);
-    const u4v* ssrc = reinterpret_cast<const u4v*>(p.runs_side + (size_t)b * nl * kRun);
-    u4v v[kPer], sv[kSPer];
+  // the q-th record of every run and the threads' records, with their row
+  // keys: every load issued before any is used (runs past the last one read
+  // it again, unused)
+  typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+  const u4v* recs = reinterpret_cast<const u4v*>(p.runs_rec + (size_t)b * nl * kRun);
+  const u2v* sides = reinterpret_cast<const u2v*>(p.runs_side + (size_t)b * nl * kRun);
+  const uint32_t k8 = tid & 7u;
+  const uint32_t qrec = p.runs_rec[((size_t)b * nl + min(tid, nl - 1u)) * kRun + p.q - 1u];
+  u4v held[4];
+  u2v held_side[4];
+  auto run_of = [&](uint32_t i) { return WIDE ? i * kHeldRuns + (tid >> 3) : tid >> 3; };
 #pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i)
-      if (tid + i * kFinishThreads < total) v[i] = src[tid + i * kFinishThreads];
-#pragma unroll
-    for (uint32_t i = 0; i < kSPer; ++i)
-      if (tid + i * kFinishThreads < stotal) sv[i] = ssrc[tid + i * kFinishThreads];
-#pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-      const uint32_t e = tid + i * kFinishThreads;
-      if (e < total) reinterpret_cast<u4v*>(lists)[(e / kV) * (kRunPitch / 4) + e % kV] = v[i];
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < kSPer; ++i) {
-      const uint32_t e = tid + i * kFinishThreads;
-      if (e < stotal) reinterpret_cast<u4v*>(lside)[(e / kSV) * (kSidePitch / 8) + e % kSV] = sv[i];
-    }
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t at = min(run_of(i), nl - 1u) * (kRun / 4) + (WIDE ? 0u : i * 8u) + k8;
+    held[i] = recs[at];
+    held_side[i] = sides[at];
   }
+  if (tid < kRuns) qth[tid] = tid < nl ? qrec : kPad;
   if (tid == 0) {
     count = 0;
     count2 = 0;
     nx = 0;
     nxr = 0;
+    if (p.m == 0) bound[0] = bound[1] = kPad - 1u;  // no such rank: every record
   }
   __syncthreads();
 
-  // Candidates: records up to R, the largest of the prefix ends (the first
-  // min(q, len) records of each run hold at least K records, so the K-th
-  // smallest is at most R).  Wave 0, lane t: runs t and t + 64; the count
-  // past the prefix scans 16 records a step.
-  if (tid < 64) {
-    uint32_t len[2], m[2], R = 0;
+  auto sum8 = [](uint32_t v) {
+    v += dev::lane_xor_bits<1>(v);
+    v += dev::lane_xor_bits<2>(v);
+    return v + dev::lane_xor_bits<4>(v);
+  };
+  // the ranks of the q-th records among themselves (records are unique; runs
+  // shorter than q hold kPad there and come last)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t l = tid + 64u * h;
-      len[h] = l < nl ? min(kRun, p.A - l * kRun) : 0u;
-      m[h] = min(p.q, len[h]);
-      if (m[h]) R = max(R, lists[l * kRunPitch + m[h] - 1]);
+  for (uint32_t i = 0; i < (WIDE ? 4u : 1u); ++i) {
+    const uint32_t l = run_of(i), mine = qth[l];
+    uint32_t below = 0;
+    for (uint32_t j = k8; j * 4u < nl; j += 8) {
+      const u4v w = reinterpret_cast<const u4v*>(qth)[j];
+      below += (w.x < mine) + (w.y < mine) + (w.z < mine) + (w.w < mine);
     }
-    R = wave_max_u32(R);
-    uint32_t c[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t* lp = lists + (tid + 64u * h) * kRunPitch;
-      const uint32_t n = len[h];
-      c[h] = m[h];  // the first m records are at most R
-      while (c[h] < n) {
-        const uint32_t c4 = c[h] & ~3u;
-        uint32_t hit = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          const uint32_t at = c4 + 4 * u;
-          const u4v v = at < n ? reinterpret_cast<const u4v*>(lp)[at / 4] : (u4v)kPad;
-          hit += (v.x <= R) + (v.y <= R) + (v.z <= R) + (v.w <= R);
-        }
-        const uint32_t before = c[h] - c4;  // records of the first vector already counted
-        const uint32_t found = hit - min(hit, before);
-        c[h] = min(c[h] + found, n);
-        if (found < 16 - before) break;
-      }
-    }
-    const uint32_t incl0 = wave_scan_u32(c[0]);
-    const uint32_t total0 = (uint32_t)__builtin_amdgcn_readlane((int)incl0, 63);
-    const uint32_t incl1 = wave_scan_u32(c[1]) + total0;
-    if (tid < nl) {
-      cnt[tid] = c[0];
-      off[tid] = incl0 - c[0];
-    }
-    if (tid + 64 < nl) {
-      cnt[tid + 64] = c[1];
-      off[tid + 64] = incl1 - c[1];
-    }
-    if (tid == 63) {
-      off[kMaxRuns] = incl1;
-      bound = R;
+    below = sum8(below);
+    if (k8 == 0 && l < nl && mine != kPad) {
+      if (below + 1u == p.m) bound[0] = mine;
+      if (below + 1u == p.m2) bound[1] = mine;
     }
   }
   __syncthreads();
-  const uint32_t C = off[kMaxRuns], Rkey = bound >> 16;
-  // eight threads per run walk its candidates
+  const uint32_t R0 = bound[0], R1 = bound[1];
+  {
+    uint32_t c0 = 0, c1 = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const u4v w = held[i];
+      c0 += (w.x <= R0) + (w.y <= R0) + (w.z <= R0) + (w.w <= R0);
+      c1 += (w.x <= R1) + (w.y <= R1) + (w.z <= R1) + (w.w <= R1);
+      if (WIDE || i == 3) {
+        const uint32_t l = run_of(i);
+        c0 = sum8(c0);
+        c1 = sum8(c1);
+        if (WIDE) {
+          for (uint32_t t = 1; t < 4 && c0 == 32u * t; ++t) {
+            const u4v x = recs[min(l, nl - 1u) * (kRun / 4) + t * 8u + k8];
+            c0 += sum8((x.x <= R0) + (x.y <= R0) + (x.z <= R0) + (x.w <= R0));
+            c1 += sum8((x.x <= R1) + (x.y <= R1) + (x.z <= R1) + (x.w <= R1));
+          }
+        }
+        if (k8 == 0) {
+          cnt[l] = l < nl ? c0 : 0u;
+          cnt2[l] = l < nl ? c1 : 0u;
+        }
+        c0 = 0;
+        c1 = 0;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    constexpr uint32_t kPer = kRuns / 64;
+    uint32_t s0 = 0, s1 = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+      s0 += cnt[tid * kPer + j];
+      s1 += cnt2[tid * kPer + j];
+    }
+    const uint32_t i0 = wave_scan_u32(s0), i1 = wave_scan_u32(s1);
+    const bool low = (uint32_t)__builtin_amdgcn_readlane((int)i1, 63) >= K;
+    uint32_t at = low ? i1 - s1 : i0 - s0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+      const uint32_t l = tid * kPer + j, n = low ? cnt2[l] : cnt[l];
+      off[l] = at;
+      cnt[l] = n;
+      at += n;
+    }
+    if (tid == 63) {
+      total = at;
+      chosen = low ? R1 : R0;
+    }
+  }
+  __syncthreads();
+  const uint32_t C = total, Rkey = chosen >> 16;
+  // each thread's candidates: record, row key, position
   auto candidates = [&](auto&& f) {
-    const uint32_t l = tid >> 3;
-    if (l < nl) {
-      const uint32_t n = cnt[l], at = off[l];
-      for (uint32_t k = tid & 7u; k < n; k += 8) f(lists[l * kRunPitch + k], lside[l * kSidePitch + k], at + k);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t l = run_of(i), n = cnt[l], at = off[l];  // n = 0 past the last run
+      auto four = [&](const u4v& w, const u2v& s, uint32_t pos) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e)
+          if (pos + e < n) f(w[e], (s[e / 2] >> (16u * (e & 1u))) & 0xffffu, at + pos + e);
+      };
+      four(held[i], held_side[i], ((WIDE ? 0u : i * 8u) + k8) * 4u);
+      if (WIDE) {
+        for (uint32_t t = 1; 32u * t < n; ++t) {
+          const uint32_t v = l * (kRun / 4) + t * 8u + k8;
+          four(recs[v], sides[v], (t * 8u + k8) * 4u);
+        }
+      }
     }
   };
   const bool few = C <= kSortCap;
@@ -1974,8 +2028,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   block_sort(sortbuf, n1, xch);
 
   if (few) {
-    // the runs are dead: the slot tables take their place
-    if (tid < C) info_slot[tid] = my_info;
+      if (tid < C) info_slot[tid] = my_info;
     if (fast && grow < G) {
 #pragma unroll
       for (uint32_t i = 0; i < kXBatch; ++i) {
@@ -2204,22 +2257,42 @@ SplitShape split_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnosti
 // scores beyond its LDS table).
 struct RunsShape {
   bool ok;
-  uint32_t runs, q, rows_per;
+  uint32_t runs, q, m, m2, rows_per;
 };
 
-RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic, int64_t image_extent) {
+RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic, int64_t image_extent, bool wide) {
   RunsShape r;
   memset(&r, 0, sizeof r);
-  if (K < 1 || K > (int64_t)kSplitMaxK || A > (int64_t)(kMaxRuns * kRun) || B > 65535 ||
+  if (K < 1 || K > (int64_t)kSplitMaxK || A > (int64_t)((wide ? kMaxRuns : kHeldRuns) * kRun) || B > 65535 ||
       image_extent >= ((int64_t)1 << 31))
     return r;
   if (!agnostic && (nc > (int64_t)kFinishThreads || K * nc > (int64_t)kPairTable)) return r;
   r.runs = (uint32_t)((A + kRun - 1) / kRun);
-  // q: the smallest prefix length whose run prefixes hold K records (every
-  // run holds kRun anchors but the last, which holds `last`)
+  // The bounds' prefix length q and rank m: m * q >= K over the runs of q or
+  // more records, at three quarters of them or, where K is most of A, as low
+  // as they allow (none: m = 0, every record).  m2: the rank up to which
+  // runs would have q records if each held a Poisson count of 1.25 K / runs.
   const int64_t last = A - (int64_t)(r.runs - 1) * kRun;
-  const int64_t q = (K + r.runs - 1) / r.runs;
-  r.q = (uint32_t)(q <= last ? q : (K - last + r.runs - 2) / (r.runs - 1));
+  for (uint32_t q = 1; q <= kRun; ++q) {
+    const int64_t have = (int64_t)r.runs - (last < (int64_t)q ? 1 : 0), m = (K + q - 1) / q;
+    if (m > have) continue;
+    r.q = q;
+    r.m = (uint32_t)m;
+    if (4 * m > 3 * have) continue;
+    break;
+  }
+  if (!r.m) {
+    r.q = 1;
+  } else {
+    const double mean = 1.25 * (double)K / r.runs;
+    double term = exp(-mean), below = 0;
+    for (uint32_t i = 0; i < r.q; ++i) {
+      below += term;
+      term *= mean / (i + 1);
+    }
+    const double rank = (1.0 - below) * r.runs;
+    r.m2 = rank < 1 ? 1 : rank > r.m ? r.m : (uint32_t)rank;
+  }
   r.rows_per = agnostic ? 0u : (uint32_t)(kFinishThreads / nc);
   r.ok = true;
   return r;
@@ -2237,11 +2310,14 @@ size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 // image_extent: elements one image of `decoded` spans (its largest offset + 1);
 // -1 when unknown (workspace queries size for the split path whenever it
 // could apply).
-WsLayout ws_layout(int64_t B, int64_t A, int64_t nc, int64_t max_det, bool agnostic, int64_t image_extent = -1) {
+// wide: images of more than kHeldRuns runs may take the two-launch selection
+// (whose workspace is larger than the other paths').
+WsLayout ws_layout(int64_t B, int64_t A, int64_t nc, int64_t max_det, bool agnostic, int64_t image_extent = -1,
+                   bool wide = true) {
   WsLayout w;
   memset(&w, 0, sizeof w);
   const int64_t K = max_det < A ? max_det : A;
-  w.two = runs_shape(B, A, nc, K, agnostic, image_extent < 0 ? 0 : image_extent);
+  w.two = runs_shape(B, A, nc, K, agnostic, image_extent < 0 ? 0 : image_extent, wide);
   if (!w.two.ok) w.split = split_shape(B, A, nc, K, agnostic, image_extent < 0 ? 0 : image_extent);
   size_t off = 0;
   w.bits1 = off; off += up256((size_t)(B * A) * 2);
@@ -2377,6 +2453,8 @@ thin_status select_run(const thin_desc* decoded, int64_t max_det, bool agn, void
     rp.K = (uint32_t)K;
     rp.runs = w.two.runs;
     rp.q = w.two.q;
+    rp.m = w.two.m;
+    rp.m2 = w.two.m2;
     rp.rows_per = w.two.rows_per;
     rp.agnostic = agn ? 1 : 0;
     rp.vec_classes = vec_classes ? 1 : 0;
@@ -2390,9 +2468,17 @@ thin_status select_run(const thin_desc* decoded, int64_t max_det, bool agn, void
     rp.info = reinterpret_cast<u4v*>(ws + w.info);
     rp.out = static_cast<uint32_t*>(out);
     rp.tr = tr;
-    hipLaunchKernelGGL(runs_kernel, dim3(rp.runs, (uint32_t)B), dim3(kRunThreads), 0, stream, rp);
+    // few runs: 512 threads a run shorten it; many: 128 leave room for more of
+    // them at once
+    if (rp.vec_classes && (int64_t)rp.runs * B >= 512)
+      hipLaunchKernelGGL(runs_kernel<kRunManyThreads>, dim3(rp.runs, (uint32_t)B), dim3(kRunManyThreads), 0, stream, rp);
+    else
+      hipLaunchKernelGGL(runs_kernel<kRunThreads>, dim3(rp.runs, (uint32_t)B), dim3(kRunThreads), 0, stream, rp);
     THIN_LAUNCH_CHECK("select_runs");
-    hipLaunchKernelGGL(finish_kernel, dim3((uint32_t)B), dim3(kFinishThreads), 0, stream, rp);
+    if (rp.runs > kHeldRuns)
+      hipLaunchKernelGGL(finish_kernel<true>, dim3((uint32_t)B), dim3(kFinishThreads), 0, stream, rp);
+    else
+      hipLaunchKernelGGL(finish_kernel<false>, dim3((uint32_t)B), dim3(kFinishThreads), 0, stream, rp);
     THIN_LAUNCH_CHECK("select_finish");
     return THIN_OK;
   }
@@ -2513,8 +2599,11 @@ extern "C" thin_status thin_detection_select(const thin_desc* decoded, int64_t m
   thin_status s = select_validate(decoded, max_det, out, trace, &skip);
   if (s != THIN_OK || skip) return s;
   const bool agn = agnostic != 0;
-  const WsLayout w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn,
-                               image_extent(decoded));
+  WsLayout w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn,
+                         image_extent(decoded));
+  if (workspace_bytes < w.total)  // room for the one-workgroup path only
+    w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn, image_extent(decoded),
+                  false);
   THIN_REQUIRE(workspace != nullptr && workspace_bytes >= w.total, THIN_ERR_WORKSPACE,
                "detection_select: workspace of %zu bytes needed, %zu given", w.total, workspace_bytes);
   THIN_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, THIN_ERR_WORKSPACE,
@@ -2564,8 +2653,11 @@ extern "C" thin_status thin_detection_select_noalloc(const thin_desc* decoded, i
   thin_status s = select_validate(decoded, max_det, out, trace, &skip);
   if (s != THIN_OK || skip) return s;
   const bool agn = agnostic != 0;
-  const WsLayout w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn,
-                               image_extent(decoded));
+  WsLayout w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn,
+                         image_extent(decoded));
+  if (w.total > (size_t)THIN_SELECT_SCRATCH_BYTES)  // the one-workgroup path needs less
+    w = ws_layout(decoded->sizes[0], decoded->sizes[1], decoded->sizes[2] - 4, max_det, agn, image_extent(decoded),
+                  false);
   THIN_REQUIRE(w.total <= (size_t)THIN_SELECT_SCRATCH_BYTES, THIN_ERR_WORKSPACE,
                "detection_select_noalloc: these sizes need %zu bytes of scratch, the static scratch holds %zu "
                "(use thin_detection_select with a workspace)",
