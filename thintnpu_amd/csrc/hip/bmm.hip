@@ -449,9 +449,9 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
 
 // The same for K <= 32 (one chunk): the block keeps its Q operand in registers
 // and walks `span` P tiles, the next tile's loads in flight under the products
-// and stores of this one.  At [128,400,32] x [128,32,400] 24.3 us (96.9 with
-// the fma chains this replaced), where the products take 9 us and the 41 MB
-// of outputs about 8.
+// and stores of this one.  At [128,400,32] x [128,32,400] 23.8 us (96.9 with
+// the fma chains this replaced): 9 us of it without products and stores, the
+// products add 11 and the stores of 41 MB 3.
 template <int W, bool PR, bool QR>
 __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   constexpr int KD = 32, R = 32 * W;
@@ -521,10 +521,11 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
       }
       sp.load(bp, vp);
     }
-    if (pr < p.P.rows && q0 + wq < p.Q.rows) {
+    const bool work = pr < p.P.rows && q0 + wq < p.Q.rows;
+    f4 acc[W][W];
+    if (work) {
       typename OP::Group gp;
       op.read(gp, ldsp + kFrom, 0);
-      f4 acc[W][W];
       bmm_call<W, true>(acc, gp, gq, 0);
       if (calls == 8u) {
 #pragma unroll
@@ -534,6 +535,16 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
         for (uint32_t s = 1; s < 7; ++s)
           if (s < calls) bmm_call<W>(acc, gp, gq, s);
       }
+    }
+    // the next tile into LDS before this one's outputs are stored: its loads
+    // and the stores are counted together, and a wait for them after the
+    // stores waits for the stores as well (24.9 against 23.9 us at
+    // [128,400,32] x [128,32,400])
+    if (more) {
+      if (K < KD) sp.trim(0, K, vp);
+      sp.store(ldsp + kTo, vp);
+    }
+    if (work) {
       if (p.y_vec && pt + 1u < p.ptiles) {
 #pragma unroll
         for (uint32_t t = 0; t < W; ++t) {
@@ -549,11 +560,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
         bmm_write<W, SP, SQ>(p, bt, acc, pr + (lane >> 4) * (4u * W), pt * R, q0 + wq, qt * R, lane);
       }
     }
-    if (more) {
-      if (K < KD) sp.trim(0, K, vp);
-      sp.store(ldsp + kTo, vp);
-      __syncthreads();
-    }
+    if (more) __syncthreads();
     ++pt;
   };
   for (;;) {
@@ -881,11 +888,12 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   THIN_REQUIRE(blocks(r) < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
   p.span = 1;
   if (fast && one) {
-    // as many P tiles a block as leave about three blocks a compute unit, in
-    // even shares (q^T k: [128,400,32] x [128,32,400] 26.1 us with one tile a
-    // block and 24.3 with all seven, [4,1600,32] x [4,32,1600] 13.7 us with up
-    // to four and 16.0 with seven)
-    const uint64_t share = blocks(r) / 800;
+    // as many P tiles a block as leave a block or two a compute unit, in even
+    // shares: a wave's fixed work is then spread over more products (q^T k
+    // [128,400,32] x [128,32,400] 23.8 us with all seven tiles a block, 25.1
+    // with two; [4,1600,32] x [4,32,1600] 12.2 us with five, 13.2 with three,
+    // 13.5 with one)
+    const uint64_t share = blocks(r) / 400;
     const uint32_t most = share < 1 ? 1u : share > 8 ? 8u : (uint32_t)share;
     const uint32_t parts = (p.ptiles + most - 1) / most;
     p.span = (p.ptiles + parts - 1) / parts;
