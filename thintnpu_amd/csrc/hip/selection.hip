@@ -18,9 +18,8 @@
 
 #include <type_traits>
 
-#include <string.h>
-
 #include <math.h>
+#include <string.h>
 
 #include <algorithm>
 #include <mutex>
@@ -1240,7 +1239,7 @@ __global__ __launch_bounds__(kSplitThreads) void merge2_kernel(SplitPlan p) {
 }
 
 // ---------------------------------------------------------------- two-launch selection
-// The selection in two launches, for one image or a few:
+// The selection in two launches, for images of up to kMaxRuns * kRun anchors:
 //
 //   runs   (grid runs x B, 512 threads): per anchor of kRun, the three
 //          smallest (key << 16 | class) over the classes; the run's
@@ -1249,7 +1248,7 @@ __global__ __launch_bounds__(kSplitThreads) void merge2_kernel(SplitPlan p) {
 //          runs_side; per anchor a 16-byte info record (box, class-max score
 //          bits and class, second key and class) -> info.
 //   finish (grid B, 1024 threads): the stage-1 candidates of the sorted runs
-//          (the prefix bound of the split kernels), sorted, while the info of
+//          (a bound by the rank of their q-th records), sorted, while the info of
 //          every candidate and the score rows of the few candidates whose
 //          third key could reach the bound are in flight; stage 2 from the K
 //          class-max pairs, the second pairs and those rows; rows packed
