@@ -173,3 +173,22 @@ def test_decode_direct_distances(gpu, xywh):
         flat = [v for hw in shapes for v in hw]
         npu = torch.ops.thin_fused.detect_decode(dist.to("npu"), scores.to("npu"), flat, strides, xywh).cpu()
     assert bits_equal(npu, capi.detect_decode(dist.to(gpu), scores.to(gpu), shapes, strides, xywh).cpu())
+
+
+@pytest.mark.parametrize("a", [7, 8, 9, 13, 16, 23, 2050, 4101])
+@pytest.mark.parametrize("nc", [1, 5])
+def test_decode_row_ends(gpu, a, nc):
+    """Class rows of any length and alignment: whole 16-byte units, every kind
+    of remainder, fewer anchors than a unit, and (the last two) more than one
+    unit per thread; into a tensor and into a view at an odd offset."""
+    from thintnpu_amd import capi
+    shapes, strides = [(1, a - 2), (1, 2)], [8.0, 16.0]
+    boxes, scores = inputs(3, nc, shapes, a)
+    want = composed(capi, gpu, boxes, scores, shapes, strides, False)
+    assert bits_equal(capi.detect_decode(boxes.to(gpu), scores.to(gpu), shapes, strides).cpu(), want.cpu())
+    wide = torch.full((3, 4 + nc, a + 5), 7.0, dtype=torch.float16, device=gpu)
+    head = torch.zeros((3, nc, a + 3), dtype=torch.float16, device=gpu)
+    head[:, :, 1:1 + a] = scores.to(gpu)
+    capi.detect_decode(boxes.to(gpu), head[:, :, 1:1 + a], shapes, strides, out=wide[:, :, 3:3 + a])
+    assert bits_equal(wide[:, :, 3:3 + a].cpu(), want.cpu())
+    assert wide[:, :, :3].eq(7).all() and wide[:, :, 3 + a:].eq(7).all()

@@ -13,6 +13,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 
 namespace thin {
 namespace {
@@ -664,7 +665,9 @@ __global__ __launch_bounds__(kThreads) void dfl_expect_rows_kernel(DflPlan p) {
 // centres (x + 0.5, y + 0.5) in fp16, anchor index = level start + y*w + x.
 // Blocks [0, box_blocks) decode boxes: a thread takes one axis (x or y) of V
 // adjacent anchors and so the box sides axis and axis+2.  The remaining blocks
-// apply the sigmoid to the class logits, 8 per thread when rows are aligned.
+// apply the sigmoid to the class logits, 8 adjacent ones at a time.  The bound
+// is HBM; at one logit a thread, which only rows of scattered anchors or fewer
+// than 8 still take, it is the issue of 2-byte accesses instead.
 constexpr int kMaxLevels = 8;
 
 struct DecodePlan {
@@ -680,12 +683,13 @@ struct DecodePlan {
   uint32_t box_units;     // B * 2 * apairs
   uint32_t box_blocks;
   uint32_t nc;
-  uint32_t svecs;         // A / VS
+  uint32_t svecs;         // A / VS, rounded up
   uint32_t score_units;   // B * nc * svecs
   FastDiv div_apairs, div_svecs, div_nc;
   int32_t xywh;
   uint32_t boxes_bytes;   // byte extent of boxes from its base (buffer-load forms)
   int32_t direct;         // boxes are the distances themselves (reg_max = 1 heads)
+  uint32_t anchors;       // A
 };
 
 __device__ __forceinline__ _Float16 h_from_bits(uint16_t b) { return __builtin_bit_cast(_Float16, b); }
@@ -698,7 +702,11 @@ constexpr uint32_t kDecodeScoreUnits = VS == 8 ? 2u : 1u;
 // LOAD 0: 64-bit pointers.  LOAD 1/2: box offsets fit 32 bits and the bins
 // are read through a buffer resource; 2 also streams the score loads and the
 // output stores (launches of at least kStreamingBytes).
-template <int VB, int VS, int LOAD>
+// ENDS (with VS 8): rows at any 2-byte alignment and of any length of at least
+// 8.  [5,186,27930] scores take 26.4 us so, 68.0 us an element at a time;
+// aligned rows keep the form without it, which is 0.5 us faster for 32 frames
+// of [80,8400] (25.1 us against 25.6).
+template <int VB, int VS, bool ENDS, int LOAD>
 __global__ __launch_bounds__(kThreads) void detect_decode_kernel(DecodePlan p) {
   // Both roles' plan fields in registers before the test of the role: they
   // then load in the same round of scalar loads as p.box_blocks, not in two
@@ -794,35 +802,44 @@ __global__ __launch_bounds__(kThreads) void detect_decode_kernel(DecodePlan p) {
     return;
   }
   // scores: two 16-byte vectors per thread (both loads issued first), or one
-  // element per thread in the unaligned form
+  // element per thread where anchors are not adjacent
   constexpr uint32_t SU = kDecodeScoreUnits<VS>;
+  typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
+  using vec = std::conditional_t<ENDS, h8u, dev::h8>;
   const uint32_t v0 = (blockIdx.x - p.box_blocks) * (kThreads * SU) + threadIdx.x;
   const _Float16* sp[SU];
   _Float16* op[SU];
+  uint32_t left[SU];  // ENDS: anchors of the row from the unit's first on
 #pragma unroll
   for (uint32_t s = 0; s < SU; ++s) {
     const uint32_t v = min(v0 + s * kThreads, p.score_units - 1);
     const uint32_t row = p.div_svecs.div(v);               // b * nc + c
     const uint32_t a0 = (v - row * p.svecs) * VS;
     const uint32_t b = p.div_nc.div(row), c = row - b * p.nc;
+    left[s] = ENDS ? p.anchors - a0 : 8u;
     sp[s] = p.scores + b * p.sb + (int64_t)c * p.sc + (int64_t)a0 * p.sa;
     op[s] = p.out + b * p.ob + (int64_t)(4 + c) * p.oc + (int64_t)a0 * p.oa;
   }
   if constexpr (VS == 8) {
-    dev::h8 x[SU];
+    vec x[SU];
 #pragma unroll
     for (uint32_t s = 0; s < SU; ++s) {
-      const dev::h8* src = reinterpret_cast<const dev::h8*>(sp[s]);
+      // a partial unit loads the row's last 8 instead, unused
+      const vec* src = reinterpret_cast<const vec*>(ENDS ? sp[s] - (8u - min(left[s], 8u)) : sp[s]);
       x[s] = LOAD == 2 ? __builtin_nontemporal_load(src) : *src;
     }
 #pragma unroll
     for (uint32_t s = 0; s < SU; ++s) {
       if (v0 + s * kThreads >= p.score_units) break;
-      dev::h8 y;
+      if (ENDS && left[s] < 8u) {
+        for (uint32_t j = 0; j < left[s]; ++j) op[s][j] = (_Float16)dev::sigmoid_fast((float)sp[s][j]);
+        continue;
+      }
+      vec y;
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = (_Float16)dev::sigmoid_fast((float)x[s][j]);
-      if constexpr (LOAD == 2) __builtin_nontemporal_store(y, reinterpret_cast<dev::h8*>(op[s]));
-      else *reinterpret_cast<dev::h8*>(op[s]) = y;
+      if constexpr (LOAD == 2) __builtin_nontemporal_store(y, reinterpret_cast<vec*>(op[s]));
+      else *reinterpret_cast<vec*>(op[s]) = y;
     }
   } else {
     if (v0 < p.score_units) op[0][0] = (_Float16)dev::sigmoid_fast((float)sp[0][0]);
@@ -1170,14 +1187,18 @@ extern "C" thin_status thin_detect_decode(const thin_desc* boxes, const thin_des
   p.direct = boxes->sizes[1] == 4 ? 1 : 0;
   const bool vb = A % 2 == 0 && p.ba == 1 && p.oa == 1 && aligned(boxes->data, 4) && aligned(out->data, 4) &&
                   p.bb % 2 == 0 && p.bc % 2 == 0 && p.ob % 2 == 0 && p.oc % 2 == 0;
-  const bool vs = A % 8 == 0 && p.sa == 1 && p.oa == 1 && aligned(scores->data, 16) && aligned(out->data, 16) &&
-                  p.sb % 8 == 0 && p.sc % 8 == 0 && p.ob % 8 == 0 && p.oc % 8 == 0;
+  const bool vs = A >= 8 && p.sa == 1 && p.oa == 1;
+  const bool ends = !(A % 8 == 0 && aligned(scores->data, 16) && aligned(out->data, 16) && p.sb % 8 == 0 &&
+                      p.sc % 8 == 0 && p.ob % 8 == 0 && p.oc % 8 == 0);
   const int VB = vb ? 2 : 1, VS = vs ? 8 : 1;
   p.apairs = (uint32_t)(A / VB);
   const uint64_t box_units = (uint64_t)B * 2 * p.apairs;
-  p.svecs = (uint32_t)(A / VS);
+  p.svecs = (uint32_t)((A + VS - 1) / VS);
+  p.anchors = (uint32_t)A;
   const uint64_t score_units = (uint64_t)B * nc * p.svecs;
-  THIN_REQUIRE(box_units < (1ull << 31) && score_units < (1ull << 31), THIN_ERR_UNSUPPORTED,
+  // (unaligned rows: the limit of one element a unit, whichever form takes them)
+  const uint64_t score_limit = vs && ends ? (uint64_t)B * nc * A : score_units;
+  THIN_REQUIRE(box_units < (1ull << 31) && score_limit < (1ull << 31), THIN_ERR_UNSUPPORTED,
                "detect_decode: tensors too large");
   p.box_units = (uint32_t)box_units;
   p.score_units = (uint32_t)score_units;
@@ -1197,16 +1218,19 @@ extern "C" thin_status thin_detect_decode(const thin_desc* boxes, const thin_des
   o32 = o32 && extent < (1ull << 32);
   p.boxes_bytes = o32 ? (uint32_t)extent : 0u;
   const int load = !o32 ? 0 : numel(out) * 2 >= kStreamingBytes ? 2 : 1;
-#define THIN_DECODE(B_, S_)                                                                                      \
+#define THIN_DECODE(B_, S_, E_)                                                                                  \
   do {                                                                                                           \
-    if (load == 2) hipLaunchKernelGGL((detect_decode_kernel<B_, S_, 2>), dim3(grid), dim3(kThreads), 0, stream, p); \
-    else if (load == 1) hipLaunchKernelGGL((detect_decode_kernel<B_, S_, 1>), dim3(grid), dim3(kThreads), 0, stream, p); \
-    else hipLaunchKernelGGL((detect_decode_kernel<B_, S_, 0>), dim3(grid), dim3(kThreads), 0, stream, p);           \
+    if (load == 2) hipLaunchKernelGGL((detect_decode_kernel<B_, S_, E_, 2>), dim3(grid), dim3(kThreads), 0, stream, p); \
+    else if (load == 1) hipLaunchKernelGGL((detect_decode_kernel<B_, S_, E_, 1>), dim3(grid), dim3(kThreads), 0, stream, p); \
+    else hipLaunchKernelGGL((detect_decode_kernel<B_, S_, E_, 0>), dim3(grid), dim3(kThreads), 0, stream, p);           \
   } while (0)
-  if (vb && vs) THIN_DECODE(2, 8);
-  else if (vb) THIN_DECODE(2, 1);
-  else if (vs) THIN_DECODE(1, 8);
-  else THIN_DECODE(1, 1);
+  if (vs && ends) {
+    if (vb) THIN_DECODE(2, 8, true);
+    else THIN_DECODE(1, 8, true);
+  } else if (vb && vs) THIN_DECODE(2, 8, false);
+  else if (vb) THIN_DECODE(2, 1, false);
+  else if (vs) THIN_DECODE(1, 8, false);
+  else THIN_DECODE(1, 1, false);
 #undef THIN_DECODE
   THIN_LAUNCH_CHECK("detect_decode");
   return THIN_OK;
