@@ -274,3 +274,38 @@ def test_blocked_widths(gpu, c0, key, tokens):
     # a range of channels that starts inside a block
     got = capi.layout_bmm(q, k, True, False, False, 0, 4, 20, 4, 20)
     assert bits_equal(got, ob.layout_bmm(qr, kr, True, False, False, 0, 4, 20, 4, 20))
+
+
+def _blocked(batch, channels, tokens, c0, g):
+    """[batch, C1, tokens, c0] of `channels` channels, the blocks filled up with NaN."""
+    x = torch.randn(batch, (channels + c0 - 1) // c0, tokens, c0, generator=g).half()
+    x[:, -1, :, (channels - 1) % c0 + 1:] = float("nan")
+    return x
+
+
+@pytest.mark.parametrize("c0", [8, 16, 32])
+@pytest.mark.parametrize("count", [9, 12, 17, 20, 23, 33, 36, 39, 131])
+def test_blocked_step_tails(gpu, c0, count):
+    """Reductions over blocked channels whose count is no multiple of 8: the
+    steps after the last whole run of 8 lie in their own block, not behind the
+    run before them.  From origin 0 and 8, with q^T k, one blocked and one
+    plain operand either way round, heads of one tensor, and 512 or more
+    64 x 64 tiles."""
+    from thintnpu_amd import capi
+    g = gen(c0 * 1000 + count)
+    for origin in (0, 8):
+        for batch, tokens in ((2, 41), (130, 70)):
+            x, y = _blocked(batch, origin + count, tokens, c0, g), _blocked(batch, origin + count, tokens, c0, g)
+            xd, yd = x.to(gpu), y.to(gpu)
+            args = (True, False, False, 0, origin, count, origin, count)
+            assert bits_equal(capi.layout_bmm(xd, yd, *args), ob.layout_bmm(x, y, *args))
+        plain = torch.randn(130, 37, count, generator=g).half()
+        args = (False, False, False, 0, 0, -1, origin, count)
+        assert bits_equal(capi.layout_bmm(plain.to(gpu), yd, *args), ob.layout_bmm(plain, y, *args))
+        right = plain.transpose(1, 2)
+        args = (True, False, False, 0, origin, count)
+        assert bits_equal(capi.layout_bmm(xd, plain.to(gpu).transpose(1, 2), *args), ob.layout_bmm(x, right, *args))
+        group = (origin + count + 31) // 32 * 32
+        heads = _blocked(1, 3 * group, 50, c0, g)
+        args = (True, False, False, 3, origin, count, origin, count)
+        assert bits_equal(capi.layout_bmm(heads.to(gpu), heads.to(gpu), *args), ob.layout_bmm(heads, heads, *args))

@@ -52,7 +52,9 @@ struct Side {
   int64_t batch;
   int64_t hop;  // bytes from a chunk of steps (bmm_kernel) or a tile of rows (bmm_short_kernel's P) to the next
   uint32_t row_origin, step_origin, row_group, step_group, rows;
-  bool steps_near;  // the smaller stride is along the steps
+  uint32_t last_run;  // first step of the last run of 8 to load: K - 8 on a plain axis, whose memory may end with the
+                      // row, the last multiple of 8 below K on a blocked one, whose blocks hold whole runs
+  bool steps_near;    // the smaller stride is along the steps
   Axis row, step;
 };
 
@@ -165,7 +167,7 @@ struct Stage {
       const int64_t row = s.row.at(ro + min(r0 + along(), s.rows - 1u));
 #pragma unroll
       for (uint32_t h = 0; h < 2; ++h)
-        off[h] = (uint32_t)(row + s.step.at(so + min(k0 + across() * 16u + 8u * h, K - 8u))) * 2u;
+        off[h] = (uint32_t)(row + s.step.at(so + min(k0 + across() * 16u + 8u * h, s.last_run))) * 2u;
     }
   }
 
@@ -178,8 +180,8 @@ struct Stage {
   }
 
   // zeroes the steps past the end (a zero product leaves every sum as it is);
-  // the run of steps across the end was loaded as the last 8
-  __device__ __forceinline__ void trim(uint32_t k0, uint32_t K, Regs& v) const {
+  // the run of steps across the end was loaded from last_run on
+  __device__ __forceinline__ void trim(const Side& s, uint32_t k0, uint32_t K, Regs& v) const {
     const h8 zero = (h8)(_Float16)0;
 #pragma unroll
     for (uint32_t u = 0; u < kLoads; ++u) {
@@ -187,10 +189,17 @@ struct Stage {
         if (k0 + along() + u * kNext >= K) v[u] = zero;
       } else {
         typedef uint64_t u2 __attribute__((ext_vector_type(2)));
-        const uint32_t k = k0 + across() * 16u + 8u * u, c = K & 7u, cut = 16u * (8u - c);
+        const uint32_t k = k0 + across() * 16u + 8u * u, c = K & 7u;  // c steps of the run across the end
         if (c && k < K && k + 8u > K) {
           const u2 d = __builtin_bit_cast(u2, v[u]);
-          const u2 r = cut < 64u ? (u2){d[0] >> cut | d[1] << (64u - cut), d[1] >> cut} : (u2){d[1] >> (cut - 64u), 0};
+          u2 r;
+          if (s.step.blk.d == 1) {  // they are the last c of the 8: to the front, zeros behind
+            const uint32_t cut = 16u * (8u - c);
+            r = cut < 64u ? (u2){d[0] >> cut | d[1] << (64u - cut), d[1] >> cut} : (u2){d[1] >> (cut - 64u), 0};
+          } else {  // the first c of the 8
+            const uint64_t keep = (1ull << 16u * (c & 3u)) - 1u;
+            r = c < 4u ? (u2){d[0] & keep, 0} : (u2){d[0], d[1] & keep};
+          }
           v[u] = __builtin_bit_cast(h8, r);
         }
         if (k >= K) v[u] = zero;
@@ -391,8 +400,8 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
   uint32_t c = 0;  // the chunk to multiply
   auto store = [&](int set, float* to, bool end) __attribute__((always_inline)) {
     if (end) {
-      sp.trim(last * KD, K, vp[set]);
-      sq.trim(last * KD, K, vq[set]);
+      sp.trim(p.P, last * KD, K, vp[set]);
+      sq.trim(p.Q, last * KD, K, vq[set]);
     }
     sp.store(to, vp[set]);
     sq.store(to + SP::kFloats, vq[set]);
@@ -487,8 +496,8 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   oq.init(wq, lane);
   float* const ldsp = lds + SQ::kFloats;
   if (K < KD) {
-    sq.trim(0, K, vq);
-    sp.trim(0, K, vp);
+    sq.trim(p.Q, 0, K, vq);
+    sp.trim(p.P, 0, K, vp);
   }
   sq.store(lds, vq);
   sp.store(ldsp, vp);
@@ -541,7 +550,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     // stores waits for the stores as well (24.9 against 23.9 us at
     // [128,400,32] x [128,32,400])
     if (more) {
-      if (K < KD) sp.trim(0, K, vp);
+      if (K < KD) sp.trim(p.P, 0, K, vp);
       sp.store(ldsp + kTo, vp);
     }
     if (work) {
@@ -879,6 +888,8 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   const bool one = s.k <= 32;  // one chunk of steps
   const uint32_t r = 32 * w, kd = (uint32_t)bmm_depth((int)w);
   const bool pr = !steps_runs(p.P), qr = !steps_runs(p.Q);
+  for (Side* x : {&p.P, &p.Q})  // (of operands with K >= 8 steps in runs)
+    x->last_run = x->step.blk.d == 1 ? (uint32_t)s.k - 8u : ((uint32_t)s.k - 1u) & ~7u;
   p.P.steps_near = unit_step(p.P.step) <= unit_step(p.P.row);
   p.Q.steps_near = unit_step(p.Q.step) <= unit_step(p.Q.row);
   const uint32_t rp = fast ? r : p.Q.rows <= 16 ? 64 : p.P.rows <= 16 ? 16 : 32, rq = fast ? r : 1024 / rp;
