@@ -309,3 +309,37 @@ def test_blocked_step_tails(gpu, c0, count):
         heads = _blocked(1, 3 * group, 50, c0, g)
         args = (True, False, False, 3, origin, count, origin, count)
         assert bits_equal(capi.layout_bmm(heads.to(gpu), heads.to(gpu), *args), ob.layout_bmm(heads, heads, *args))
+
+
+@pytest.mark.parametrize("c0", [8, 24, 40, 64, 128])
+@pytest.mark.parametrize("channels", [20, 100])
+def test_blocked_axis_forms(gpu, c0, channels):
+    """Channel blocks of widths that do and do not divide a chunk of steps or
+    a tile of rows, as rows of either operand (the last run of rows partial)
+    and as steps, with one tile a block and several."""
+    from thintnpu_amd import capi
+    g = gen(c0 + channels)
+    for batch, tokens in ((2, 131), (2, 24), (450, 24)):
+        x = _blocked(batch, channels, tokens, c0, g)
+        rows = torch.randn(batch, tokens, 70, generator=g).half()
+        args = (False, False, False, 0, 0, channels)
+        assert bits_equal(capi.layout_bmm(x.to(gpu), rows.to(gpu), *args), ob.layout_bmm(x, rows, *args))
+        rows = torch.randn(batch, 70, tokens, generator=g).half()
+        args = (False, True, False, 0, 0, -1, 0, channels)
+        assert bits_equal(capi.layout_bmm(rows.to(gpu), x.to(gpu), *args), ob.layout_bmm(rows, x, *args))
+    args = (True, False, False, 0, 0, channels, 0, channels)
+    for batch, tokens in ((2, 131), (130, 70)):
+        x = _blocked(batch, channels, tokens, c0, g)
+        assert bits_equal(capi.layout_bmm(x.to(gpu), x.to(gpu), *args), ob.layout_bmm(x, x, *args))
+
+
+@pytest.mark.parametrize("batch", [500, 520])
+@pytest.mark.parametrize("rows,k", [(33, 20), (49, 40), (63, 130)])
+def test_partial_rows_by_batch(gpu, batch, rows, k):
+    """Row-contiguous operands of one 64-row tile that ends in a partial run,
+    on both sides of the batch from which 64 x 64 tiles fill the device."""
+    from thintnpu_amd import capi
+    a = torch.randn(batch, k, rows, generator=gen(rows)).half().transpose(1, 2)
+    b = torch.randn(batch, k, rows, generator=gen(k)).half()
+    ad = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+    assert bits_equal(capi.bmm(ad, b.to(gpu)), ob.sequential_bmm(a, b))

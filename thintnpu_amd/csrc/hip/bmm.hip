@@ -54,6 +54,7 @@ struct Side {
   uint32_t row_origin, step_origin, row_group, step_group, rows;
   uint32_t last_run;  // first step of the last run of 8 to load: K - 8 on a plain axis, whose memory may end with the
                       // row, the last multiple of 8 below K on a blocked one, whose blocks hold whole runs
+  uint32_t last_rows, early;  // the same of the runs of 8 rows; rows by which the last tile starts early for it
   bool steps_near;    // the smaller stride is along the steps
   Axis row, step;
 };
@@ -72,6 +73,7 @@ struct BmmPlan {
   uint32_t span;      // bmm_short_kernel: P tiles per block,
   int64_t yhop;       // and output elements from one to the next
   uint32_t ptiles;
+  uint32_t walk;      // blocks of an axis do not divide a chunk (a tile): offsets anew for each, no hops
   FastDiv pblocks, qtiles;
 };
 
@@ -159,7 +161,7 @@ struct Stage {
   __device__ __forceinline__ void aim(const Side& s, uint32_t bt, uint32_t r0, uint32_t k0, uint32_t K) {
     const uint32_t ro = s.row_origin + bt * s.row_group, so = s.step_origin + bt * s.step_group;
     if constexpr (RF) {
-      const int64_t row = s.row.at(ro + min(r0 + across() * 8u, s.rows - 8u));
+      const int64_t row = s.row.at(ro + min(r0 + across() * 8u, s.last_rows));
 #pragma unroll
       for (uint32_t u = 0; u < kPer; ++u)
         off[u] = (uint32_t)(row + s.step.at(so + min(k0 + along() + u * kNext, K - 1u))) * 2u;
@@ -312,12 +314,13 @@ __device__ __forceinline__ void bmm_write(const BmmPlan& p, uint32_t bt, const f
   }
 }
 
-// First row of a tile: the last tile of a row-major operand whose rows are no
-// multiple of 8 starts up to 7 rows early, so that its rows are whole runs
-// (the rows it shares with the tile before are not written).
+// First row of a tile: the last tile of an operand whose rows lie on a plain
+// axis and are no multiple of 8 starts up to 7 rows early, so that its rows
+// are whole runs (the rows it shares with the tile before are not written).
+// The blocks of a blocked axis hold whole runs.
 template <bool RF>
-__device__ __forceinline__ uint32_t tile_row(uint32_t tile, uint32_t tiles, uint32_t r, uint32_t rows) {
-  return RF && tile + 1u == tiles ? tile * r - ((0u - rows) & 7u) : tile * r;
+__device__ __forceinline__ uint32_t tile_row(const Side& s, uint32_t tile, uint32_t tiles, uint32_t r) {
+  return RF && tile + 1u == tiles ? tile * r - s.early : tile * r;
 }
 
 template <int B>
@@ -349,7 +352,7 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
   const uint32_t rest = p.pblocks.div(blockIdx.x), pt = blockIdx.x - rest * p.pblocks.d;
   const uint32_t bt = p.qtiles.div(rest), qt = rest - bt * p.qtiles.d;
   const uint32_t K = p.k;
-  const uint32_t p0 = tile_row<PR>(pt, p.ptiles, R, p.P.rows), q0 = tile_row<QR>(qt, p.qtiles.d, R, p.Q.rows);
+  const uint32_t p0 = tile_row<PR>(p.P, pt, p.ptiles, R), q0 = tile_row<QR>(p.Q, qt, p.qtiles.d, R);
   const uint32_t last = (K - 1u) / KD;  // the last chunk, whole or not
 
   SP sp;
@@ -365,9 +368,9 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
   // which nothing stores: a test around the loads would leave the waits
   // without a count of the loads behind the one they wait for
   auto load = [&](int set) __attribute__((always_inline)) {
-    if (n == last) {
-      sp.aim(p.P, bt, p0, last * KD, K);
-      sq.aim(p.Q, bt, q0, last * KD, K);
+    if (n == last || (p.walk && n < last)) {
+      sp.aim(p.P, bt, p0, n * KD, K);
+      sq.aim(p.Q, bt, q0, n * KD, K);
       bp = SP::base(p.P, bt);
       bq = SQ::base(p.Q, bt);
     }
@@ -473,7 +476,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   const uint32_t rest = p.pblocks.div(blockIdx.x), pb = blockIdx.x - rest * p.pblocks.d;
   const uint32_t bt = p.qtiles.div(rest), qt = rest - bt * p.qtiles.d;
   const uint32_t K = p.k;
-  const uint32_t q0 = tile_row<QR>(qt, p.qtiles.d, R, p.Q.rows);
+  const uint32_t q0 = tile_row<QR>(p.Q, qt, p.qtiles.d, R);
   uint32_t pt = pb * p.span;
   const uint32_t pend = min(pt + p.span, p.ptiles);
 
@@ -482,7 +485,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   typename SP::Regs vp;
   typename SQ::Regs vq;
   const char* bp = SP::base(p.P, bt);
-  uint32_t p0 = tile_row<PR>(pt, p.ptiles, R, p.P.rows);
+  uint32_t p0 = tile_row<PR>(p.P, pt, p.ptiles, R);
   sp.aim(p.P, bt, p0, 0, K);
   sq.aim(p.Q, bt, q0, 0, K);
   sq.load(SQ::base(p.Q, bt), vq);
@@ -521,8 +524,8 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     const bool more = pt + 1u < pend;
     const uint32_t pr = p0 + wp;
     if (more) {
-      p0 = tile_row<PR>(pt + 1u, p.ptiles, R, p.P.rows);
-      if (pt + 2u == p.ptiles) {
+      p0 = tile_row<PR>(p.P, pt + 1u, p.ptiles, R);
+      if (pt + 2u == p.ptiles || p.walk) {
         sp.aim(p.P, bt, p0, 0, K);
         bp = SP::base(p.P, bt);
       } else {
@@ -869,27 +872,31 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   // over four times as many waves
   auto blocks = [&](uint64_t r) { return (uint64_t)s.batch * ((p.P.rows + r - 1) / r) * ((p.Q.rows + r - 1) / r); };
   uint32_t w = blocks(64) >= 512 ? 2 : 1;
-  // whole 16-byte runs along the steps, else along the rows (rows of a plain
-  // axis may end in a partial run: the last tile then starts early, which
-  // takes a tile before it); the kernels' lane offsets are 32-bit
+  // 16-byte runs along the steps, else along the rows (rows of a plain axis
+  // may end in a partial run: the last tile then starts early, which takes a
+  // tile before it); the kernels' lane offsets are 32-bit
   auto steps_runs = [&](const Side& x) { return s.k >= 8 && runs_of(x.step, x.step_origin, x.step_group, 8); };
   auto rows_runs = [&](const Side& x) {
     return runs_of(x.row, x.row_origin, x.row_group, 8) &&
-           (x.rows % 8 == 0 || (x.row.blk.d == 1 && x.rows > 32u * w));
+           (x.row.blk.d != 1 || x.rows % 8 == 0 || x.rows > 32u * w);
   };
   auto near = [](const thin_desc* d) {
     int64_t extent = 0;
     for (int i = 1; i < d->rank; ++i) extent += (d->sizes[i] - 1) * d->strides[i];
     return extent < ((int64_t)1 << 30);
   };
-  const bool fast = (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)) && near(a) && near(b) &&
-                    32 % p.P.row.blk.d == 0 && 32 % p.P.step.blk.d == 0 && 32 % p.Q.step.blk.d == 0;
+  auto loads = [&] { return (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)); };
+  if (w == 2 && !loads()) w = 1;  // rows that end in a partial run and fill one tile of 64, but not of 32
+  const bool fast = loads() && near(a) && near(b);
   if (!fast) w = 1;
   const bool one = s.k <= 32;  // one chunk of steps
   const uint32_t r = 32 * w, kd = (uint32_t)bmm_depth((int)w);
   const bool pr = !steps_runs(p.P), qr = !steps_runs(p.Q);
-  for (Side* x : {&p.P, &p.Q})  // (of operands with K >= 8 steps in runs)
+  for (Side* x : {&p.P, &p.Q}) {  // (of operands with K >= 8 steps, or with 8 or more rows, in runs)
     x->last_run = x->step.blk.d == 1 ? (uint32_t)s.k - 8u : ((uint32_t)s.k - 1u) & ~7u;
+    x->last_rows = x->row.blk.d == 1 ? x->rows - 8u : (x->rows - 1u) & ~7u;
+    x->early = x->row.blk.d == 1 ? (0u - x->rows) & 7u : 0u;
+  }
   p.P.steps_near = unit_step(p.P.step) <= unit_step(p.P.row);
   p.Q.steps_near = unit_step(p.Q.step) <= unit_step(p.Q.row);
   const uint32_t rp = fast ? r : p.Q.rows <= 16 ? 64 : p.P.rows <= 16 ? 16 : 32, rq = fast ? r : 1024 / rp;
@@ -908,9 +915,11 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
     const uint32_t most = share < 1 ? 1u : share > 8 ? 8u : (uint32_t)share;
     const uint32_t parts = (p.ptiles + most - 1) / most;
     p.span = (p.ptiles + parts - 1) / parts;
+    p.walk = r % p.P.row.blk.d != 0;
     p.P.hop = (int64_t)(r / p.P.row.blk.d) * p.P.row.outer * 2;
     p.yhop = (int64_t)(r / p.yp.blk.d) * p.yp.outer;
   } else if (fast) {
+    p.walk = kd % p.P.step.blk.d != 0 || kd % p.Q.step.blk.d != 0;
     p.P.hop = (int64_t)(kd / p.P.step.blk.d) * p.P.step.outer * 2;
     p.Q.hop = (int64_t)(kd / p.Q.step.blk.d) * p.Q.step.outer * 2;
   }
