@@ -343,3 +343,24 @@ def test_partial_rows_by_batch(gpu, batch, rows, k):
     b = torch.randn(batch, k, rows, generator=gen(k)).half()
     ad = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
     assert bits_equal(capi.bmm(ad, b.to(gpu)), ob.sequential_bmm(a, b))
+
+
+@pytest.mark.parametrize("batch,m,n", [(3, 1, 5), (2, 40, 70), (700, 8, 65), (650, 16, 33), (650, 17, 33), (2100, 5, 70)])
+@pytest.mark.parametrize("k", [1, 8, 21, 32, 33, 40, 64, 77, 136, 520, 528])
+def test_columns_in_vectors(gpu, batch, m, n, k):
+    """Columns of b in aligned vectors along k, at sizes on both sides of the
+    choice between chains of fmas and matrix tiles: one to four rows a wave,
+    reductions around the staging rounds, rows of a adjacent (gathered below
+    8, which leaves the tiled chains) or not, columns a line apart or not."""
+    from thintnpu_amd import capi
+    if batch * m * n * k > 700 * 16 * 65 * 136:
+        batch = 2
+    g = gen(batch + m + n + k)
+    pitch = (k + 7) // 8 * 8
+    store = torch.randn(batch, n, pitch, generator=g).half()
+    b, bd = store[:, :, :k].transpose(1, 2), store.to(gpu)[:, :, :k].transpose(1, 2)
+    a = torch.randn(batch, m, k, generator=g).half()
+    expect = ob.sequential_bmm(a, b)
+    assert bits_equal(capi.bmm(a.to(gpu), bd), expect)
+    rows = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+    assert bits_equal(capi.bmm(rows, bd), expect)

@@ -42,6 +42,9 @@ struct Mat {
   int64_t batch;
   uint32_t row_origin, col_origin, row_group, col_group;
   Axis row, col;
+  __device__ __forceinline__ int64_t at(uint32_t b, uint32_t r, uint32_t c) const {
+    return (int64_t)b * batch + row.at(r + row_origin + b * row_group) + col.at(c + col_origin + b * col_group);
+  }
 };
 
 // ---------------------------------------------------------------- matrix-core product
@@ -662,7 +665,289 @@ void launch_bmm(const BmmPlan& p, bool pr, bool qr, uint32_t grid, hipStream_t s
   else launch_form<SHORT, W, false, false>(p, grid, stream);
 }
 
+// ---------------------------------------------------------------- chains on the VALU
+// A chain of fmas per output, a lane to an output column, for products that
+// leave the matrix tiles mostly empty (few rows of a, short reductions, many
+// batch entries) or that only the gather could load: b's columns must run
+// along k in aligned 16-byte vectors.  The dispatch holds both sides'
+// measurements.
+constexpr uint32_t kChainCols = 64;  // one output column per lane
+
+struct ChainPlan {
+  Mat a, b, y;  // a: [batch, m, k], b: [batch, k, n], y: [batch, m, n]
+  uint32_t m, n, k;
+  uint32_t mtiles, ntiles;
+  bool a_kfast;  // stage a along k (its smaller stride is on k)
+  // bytes from b.p to the end of its storage, vectors per contiguous run along
+  // k (0 = one run) and the byte jump after a run
+  uint32_t b_bytes, b_vrun, b_vjump;
+  FastDiv div_mt, div_nt;  // block index -> (batch, row tile, column tile)
+};
+
+// Lane j owns output column j and streams that column from memory with 16-byte
+// loads.  A block is one wave; it stages its RM rows of a in LDS as fp32
+// (KS * 64 steps at a time) and each reduction step is RM fmas on LDS
+// broadcasts.  The column is read in rounds of RV vectors (8 steps each): the
+// first round is issued before the rows of a are staged, each later round
+// loads while the previous one is consumed, and a whole round is consumed by
+// straight-line code so that the LDS reads of one vector overlap the fmas of
+// the previous one.  KS and RV are sized to K so that short reductions issue
+// no surplus loads.
+template <int RM, int KS, int RV>
+__global__ __launch_bounds__(64) void chain_stream_kernel(ChainPlan p) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  constexpr uint32_t kDepth = KS * 64;  // steps of a staged per round (a multiple of 8 * RV)
+  __shared__ __attribute__((aligned(16))) float As[RM][kDepth];
+  const uint32_t lane = threadIdx.x;
+  uint32_t t = blockIdx.x;
+  const uint32_t q = p.div_nt.div(t), nt = t - q * p.ntiles;  // no integer division sequence
+  const uint32_t bt = p.div_mt.div(q), mt = q - bt * p.mtiles;
+  const uint32_t i0 = mt * RM, j = nt * kChainCols + lane;
+  const _Float16* bcol = p.b.p + (int64_t)bt * p.b.batch +
+                         p.b.col.at(min(j, p.n - 1) + p.b.col_origin + bt * p.b.col_group);
+  const uint32_t rbase = p.b.row_origin + bt * p.b.row_group;
+  // vector v of the column holds steps [8v, 8v + 8).  Loads go through a
+  // buffer resource: the lane's column start is the vector offset, the step
+  // offset is uniform (a scalar register) and advances by 16 bytes per vector
+  // plus the run jump at each run end, so addressing costs a few scalar
+  // operations per vector.  Loads past the last whole vector re-read it and
+  // are not consumed.
+  const uint32_t nvec = p.k / 8;
+  const __amdgpu_buffer_rsrc_t brsrc = dev::buffer_rsrc(p.b.p, p.b_bytes);
+  const uint32_t bvoff = (uint32_t)(bcol - p.b.p) * 2u;
+  uint32_t bsoff = (uint32_t)p.b.row.at(rbase) * 2u;
+  uint32_t rpos = p.b_vrun ? (rbase - p.b.row.blk.div(rbase) * p.b.row.blk.d) / 8u : 0u;
+  uint32_t vaddr = 0;  // vector whose offset bsoff holds
+  auto load_round = [&](h8 (&buf)[RV]) {
+#pragma unroll
+    for (int v = 0; v < RV; ++v) {
+      buf[v] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bvoff, bsoff, 0));
+      if (vaddr + 1 < nvec) {
+        ++vaddr;
+        bsoff += 16u;
+        if (p.b_vrun && ++rpos == p.b_vrun) {
+          rpos = 0;
+          bsoff += p.b_vjump;
+        }
+      }
+    }
+  };
+  h8 cur[RV], nxt[RV];
+  if (nvec) load_round(cur);
+
+  float acc[RM];
+#pragma unroll
+  for (int r = 0; r < RM; ++r) acc[r] = 0.f;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  // rows' steps kk..kk+7 of the staged a
+  auto read_a = [&](f4 (&a)[RM][2], uint32_t kk) {
+#pragma unroll
+    for (int r = 0; r < RM; ++r) {
+      a[r][0] = *reinterpret_cast<const f4*>(&As[r][kk]);
+      a[r][1] = *reinterpret_cast<const f4*>(&As[r][kk + 4]);
+    }
+  };
+  auto fmas = [&](const f4 (&a)[RM][2], const h8& v) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float bv = (float)v[q];
+#pragma unroll
+      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(a[r][q / 4][q % 4], bv, acc[r]);
+    }
+  };
+  auto consume = [&](const h8& v, uint32_t kk) {
+    f4 a[RM][2];
+    read_a(a, kk);
+    fmas(a, v);
+  };
+  uint32_t vnext = 0;  // first vector not yet consumed (a multiple of RV between rounds)
+  for (uint32_t k0 = 0; k0 < p.k; k0 += kDepth) {
+    const uint32_t kc = min(kDepth, p.k - k0);
+    if (k0) __syncthreads();  // the previous round's rows are no longer read
+    {
+      // every load of the round in flight at once: clamped addresses, then
+      // predicated LDS stores
+      int64_t colpart[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        colpart[s] = p.a.col.at(k0 + min(lane + s * 64u, kc - 1) + p.a.col_origin + bt * p.a.col_group);
+      _Float16 av[RM][KS];
+#pragma unroll
+      for (int r = 0; r < RM; ++r) {
+        const _Float16* row = p.a.p + (int64_t)bt * p.a.batch +
+                              p.a.row.at(min(i0 + r, p.m - 1) + p.a.row_origin + bt * p.a.row_group);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) av[r][s] = row[colpart[s]];
+      }
+#pragma unroll
+      for (int r = 0; r < RM; ++r)
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          if (lane + s * 64u < kc) As[r][lane + s * 64] = (float)av[r][s];
+    }
+    __syncthreads();
+    const uint32_t vend = min(nvec, (k0 + kc) / 8);  // whole vectors inside this round
+    // whole rounds: straight-line code
+    while (vnext + RV <= vend) {
+      const bool more = vnext + RV < nvec;
+      if (more) load_round(nxt);
+      // the a steps of vector v + 1 are read while vector v's fmas run
+      f4 a0[RM][2], a1[RM][2];
+      const uint32_t kb = vnext * 8 - k0;
+      read_a(a0, kb);
+#pragma unroll
+      for (int v = 0; v < RV; v += 2) {
+        read_a(a1, kb + (v + 1) * 8);
+        fmas(a0, cur[v]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (v + 2 < RV) read_a(a0, kb + (v + 2) * 8);
+        fmas(a1, cur[v + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (more) {
+#pragma unroll
+        for (int v = 0; v < RV; ++v) cur[v] = nxt[v];
+      }
+      vnext += RV;
+    }
+    // the last, partial round
+    if (vnext < vend) {
+#pragma unroll
+      for (int v = 0; v < RV; ++v)
+        if (vnext + v < vend) consume(cur[v], (vnext + v) * 8 - k0);
+      vnext = vend;
+    }
+    // steps past the last whole vector
+    for (uint32_t kk = max(k0, nvec * 8); kk < k0 + kc; ++kk) {
+      const float bv = (float)bcol[p.b.row.at(rbase + kk)];
+#pragma unroll
+      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[r][kk - k0], bv, acc[r]);
+    }
+  }
+  if (j >= p.n) return;
+#pragma unroll
+  for (int r = 0; r < RM; ++r) {
+    const uint32_t i = i0 + r;
+    if (i < p.m) p.y.p[p.y.at(bt, i, j)] = (_Float16)acc[r];
+  }
+}
+
+// Columns of b at least a cache line apart (the probabilities of v p^T: each
+// column is a row of p): a lane that streams its own column touches a
+// different line per lane and instruction, which saturates the L1 tag lookups.
+// Here a block of 4 waves computes 4 * RM rows x 64 columns and loads b in
+// kTileDepth-step chunks with 8 lanes per column (one 128-byte line per 8
+// lanes), keeps them in LDS as fp16 step pairs, and each lane reads its column
+// two steps at a time.  The next chunk is loaded into registers while the
+// current one is consumed.  K % 8 == 0.  A dependent fp32 fma takes about 32
+// cycles, which bounds a chain however it is tiled.
+constexpr uint32_t kTileDepth = 64;
+
+template <int RM>
+__global__ __launch_bounds__(kBmmThreads) void chain_tile_kernel(ChainPlan p) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  constexpr uint32_t TM = 4 * RM;
+  constexpr uint32_t kAPitch = TM + 4;
+  constexpr uint32_t kBPitch = kChainCols + 1;  // in step pairs
+  constexpr uint32_t kAPer = TM * kTileDepth / kBmmThreads;  // a elements per thread per chunk
+  __shared__ __attribute__((aligned(16))) float As[kTileDepth][kAPitch];
+  __shared__ h2 Bs[kTileDepth / 2][kBPitch];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  uint32_t t = blockIdx.x;
+  const uint32_t nt = t % p.ntiles;
+  t /= p.ntiles;
+  const uint32_t mt = t % p.mtiles;
+  const uint32_t bt = t / p.mtiles;
+  const uint32_t i0 = mt * TM, j0 = nt * kChainCols;
+
+  // b: thread handles vectors e = tid + 256 s: column jj = e / 8, steps
+  // 8 * (e % 8) .. + 8 of the chunk
+  const __amdgpu_buffer_rsrc_t brsrc = dev::buffer_rsrc(p.b.p, p.b_bytes);
+  const uint32_t rbase = p.b.row_origin + bt * p.b.row_group;
+  uint32_t bvoff[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const uint32_t jj = (tid + s * kBmmThreads) / 8u;
+    bvoff[s] = (uint32_t)((int64_t)bt * p.b.batch +
+                          p.b.col.at(min(j0 + jj, p.n - 1) + p.b.col_origin + bt * p.b.col_group)) * 2u;
+  }
+  const uint32_t kv = tid % 8u;
+  h8 bv[2];
+  _Float16 av[kAPer];
+  auto load_chunk = [&](uint32_t k0, uint32_t kc) {
+    // vectors past the chunk's end re-read its last vector (never consumed)
+    const uint32_t kk = k0 + min(kv * 8u, kc - 8u);
+    const uint32_t soff = (uint32_t)p.b.row.at(rbase + kk) * 2u;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      bv[s] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, bvoff[s] + soff, 0, 0));
+#pragma unroll
+    for (uint32_t s = 0; s < kAPer; ++s) {
+      const uint32_t e = tid + s * kBmmThreads;
+      const uint32_t kk2 = p.a_kfast ? e % kTileDepth : e / TM;
+      const uint32_t ii = p.a_kfast ? e / kTileDepth : e % TM;
+      av[s] = p.a.p[p.a.at(bt, min(i0 + ii, p.m - 1), k0 + min(kk2, kc - 1))];
+    }
+  };
+  auto store_chunk = [&]() {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const uint32_t jj = (tid + s * kBmmThreads) / 8u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) Bs[kv * 4 + q][jj] = (h2){bv[s][2 * q], bv[s][2 * q + 1]};
+    }
+#pragma unroll
+    for (uint32_t s = 0; s < kAPer; ++s) {
+      const uint32_t e = tid + s * kBmmThreads;
+      const uint32_t kk2 = p.a_kfast ? e % kTileDepth : e / TM;
+      const uint32_t ii = p.a_kfast ? e / kTileDepth : e % TM;
+      As[kk2][ii] = (float)av[s];
+    }
+  };
+
+  float acc[RM];
+#pragma unroll
+  for (int r = 0; r < RM; ++r) acc[r] = 0.f;
+  load_chunk(0, min(kTileDepth, p.k));
+  for (uint32_t k0 = 0; k0 < p.k; k0 += kTileDepth) {
+    const uint32_t kc = min(kTileDepth, p.k - k0);
+    store_chunk();
+    __syncthreads();
+    if (k0 + kTileDepth < p.k) load_chunk(k0 + kTileDepth, min(kTileDepth, p.k - k0 - kTileDepth));
+#pragma unroll 4
+    for (uint32_t k2 = 0; k2 < kc / 2; ++k2) {
+      const h2 b = Bs[k2][lane];
+      const float b0 = (float)b[0], b1 = (float)b[1];
+#pragma unroll
+      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[2 * k2][wave * RM + r], b0, acc[r]);
+#pragma unroll
+      for (int r = 0; r < RM; ++r) acc[r] = __builtin_fmaf(As[2 * k2 + 1][wave * RM + r], b1, acc[r]);
+    }
+    __syncthreads();
+  }
+  const uint32_t j = j0 + lane;
+  if (j >= p.n) return;
+#pragma unroll
+  for (int r = 0; r < RM; ++r) {
+    const uint32_t i = i0 + wave * RM + r;
+    if (i < p.m) p.y.p[p.y.at(bt, i, j)] = (_Float16)acc[r];
+  }
+}
+
 // ---------------------------------------------------------------- host
+
+// b's columns run contiguously along k in 16-byte aligned groups of 8: unit
+// step along k (a plain axis of stride 1, or a blocked axis of in-block stride
+// 1 whose block is a multiple of 8 and whose block stride keeps 8-alignment),
+// 8-aligned column, batch and group offsets, a 16-byte aligned base.
+bool streamable_b(const Mat& b) {
+  const Axis& k = b.row;
+  const bool unit = (k.blk.d == 1 && k.outer == 1) || (k.blk.d % 8 == 0 && k.inner == 1 && k.outer % 8 == 0);
+  const bool cols = b.col.outer % 8 == 0 && (b.col.blk.d == 1 || b.col.inner % 8 == 0);
+  return unit && cols && reinterpret_cast<uintptr_t>(b.p) % 16 == 0 && b.batch % 8 == 0 && b.row_origin % 8 == 0 &&
+         b.row_group % 8 == 0;
+}
 
 // Runs of `n` consecutive indexes from multiples of n are adjacent in memory:
 // a plain axis of stride 1, or a blocked axis of in-block stride 1 whose
@@ -772,6 +1057,72 @@ thin_status check_out(const thin_desc* out, const BmmShape& s, const thin_bmm_la
                  THIN_ERR_INVALID, "bmm: blocked out must be [%lld, %lld, %lld, 16]", (long long)lead,
                  (long long)c1, (long long)s.n);
   }
+  return THIN_OK;
+}
+
+template <int RM>
+void launch_stream(const ChainPlan& p, uint32_t grid, hipStream_t stream) {
+  if (p.k <= 32)
+    hipLaunchKernelGGL((chain_stream_kernel<RM, 1, 4>), dim3(grid), dim3(64), 0, stream, p);
+  else if (p.k <= 64)
+    hipLaunchKernelGGL((chain_stream_kernel<RM, 1, 8>), dim3(grid), dim3(64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((chain_stream_kernel<RM, 8, 8>), dim3(grid), dim3(64), 0, stream, p);
+}
+
+// The product as chains; a and b as in thin_layout_bmm, b streamable and of
+// b_extent elements.
+thin_status launch_chains(const Mat& a, const Mat& b, int64_t b_extent, const BmmShape& s, const thin_desc* out,
+                          const thin_bmm_layout* L, hipStream_t stream) {
+  ChainPlan p;
+  memset(&p, 0, sizeof p);
+  p.a = a;
+  p.b = b;
+  Mat& y = p.y;
+  y.p = static_cast<_Float16*>(out->data);
+  y.batch = L->blocked_output && L->groups ? 0 : out->strides[0];
+  y.row = L->blocked_output ? make_axis(16, out->strides[1], out->strides[3]) : make_axis(1, out->strides[1], 0);
+  y.col = make_axis(1, out->strides[2], 0);
+  y.row_group = L->blocked_output && L->groups ? (uint32_t)s.m : 0u;  // head b's channels are packed from b * m on
+  p.m = (uint32_t)s.m;
+  p.n = (uint32_t)s.n;
+  p.k = (uint32_t)s.k;
+  p.a_kfast = unit_step(a.col) <= unit_step(a.row);
+  p.ntiles = (uint32_t)((s.n + kChainCols - 1) / kChainCols);
+  p.b_bytes = (uint32_t)(b_extent * 2);
+  p.b_vrun = b.row.blk.d == 1 ? 0u : b.row.blk.d / 8u;
+  p.b_vjump = b.row.blk.d == 1 ? 0u : (uint32_t)((b.row.outer - b.row.blk.d) * 2);
+  auto tiles = [&](int rows) { return (uint64_t)s.batch * ((s.m + rows - 1) / rows) * p.ntiles; };
+  if (p.k % 8 == 0 && b.col.blk.d == 1 && b.col.outer >= 64) {
+    // the tallest tile that leaves every SIMD about a wave
+    const int rm = tiles(16) * 4 >= 1024 ? 4 : tiles(8) * 4 >= 1024 ? 2 : 1;
+    p.mtiles = (uint32_t)((s.m + 4 * rm - 1) / (4 * rm));
+    const uint64_t grid = tiles(4 * rm);
+    THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
+    if (rm == 4)
+      hipLaunchKernelGGL(chain_tile_kernel<4>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
+    else if (rm == 2)
+      hipLaunchKernelGGL(chain_tile_kernel<2>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
+    else
+      hipLaunchKernelGGL(chain_tile_kernel<1>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
+    THIN_LAUNCH_CHECK("chain_tile_kernel");
+    return THIN_OK;
+  }
+  // rows per wave: 2; 1 when that leaves under half a wave per SIMD, 4 when it
+  // would queue more than 8 waves per SIMD
+  const int rm = tiles(2) < 512 ? 1 : tiles(2) > 8192 ? 4 : 2;
+  p.mtiles = (uint32_t)((s.m + rm - 1) / rm);
+  p.div_mt = FastDiv::make(p.mtiles);
+  p.div_nt = FastDiv::make(p.ntiles);
+  const uint64_t grid = tiles(rm);
+  THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
+  if (rm == 4)
+    launch_stream<4>(p, (uint32_t)grid, stream);
+  else if (rm == 2)
+    launch_stream<2>(p, (uint32_t)grid, stream);
+  else
+    launch_stream<1>(p, (uint32_t)grid, stream);
+  THIN_LAUNCH_CHECK("chain_stream_kernel");
   return THIN_OK;
 }
 
@@ -888,6 +1239,27 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   auto loads = [&] { return (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)); };
   if (w == 2 && !loads()) w = 1;  // rows that end in a partial run and fill one tile of 64, but not of 32
   const bool fast = loads() && near(a) && near(b);
+  // Where b's columns come in aligned vectors, the chains on the VALU take what
+  // only the gather could load (v p^T of 32 channels in blocks of 4, 1600
+  // tokens: 25 us against 49) and products that leave the matrix tiles empty:
+  // - short reductions with few rows ([8000,2,8] x [8000,8,4]: 5.9 us against
+  //   20) or few tiles ([16,32,8] x [16,8,96]: 3.0 against 3.5; the two meet
+  //   at about 128 tiles);
+  // - up to 16 rows, half a tile, in enough blocks that throughput counts
+  //   ([1500,16,64] x [1500,64,48]: 1.4x; [256,16,64] x [256,64,48], 512
+  //   blocks: 0.9x), longer reductions only where columns leave tiles partly
+  //   empty too ([1500,16,136]: n = 32 0.92x, n = 48 1.2x).
+  // From 24 rows on the matrix tiles are faster at every size measured.
+  const uint64_t tiles = blocks(32);
+  auto sparse = [&] {
+    if (s.k <= 32) return s.m <= 8 || tiles < 128;
+    return s.m <= 16 && tiles >= 640 && (s.k <= 64 || (s.n > 32 && s.k <= 512));
+  };
+  int64_t b_extent = 1;  // elements from b's data pointer to its last element, + 1
+  for (int d = 0; d < b->rank; ++d) b_extent += (b->sizes[d] - 1) * b->strides[d];
+  // (a launch holds 2^32 threads: 2^24 blocks of the matrix kernels)
+  if (streamable_b(bm) && b_extent * 2 < ((int64_t)1 << 31) && (!fast || sparse() || tiles >= ((uint64_t)1 << 24)))
+    return launch_chains(am, bm, b_extent, s, out, layout, stream);
   if (!fast) w = 1;
   const bool one = s.k <= 32;  // one chunk of steps
   const uint32_t r = 32 * w, kd = (uint32_t)bmm_depth((int)w);
