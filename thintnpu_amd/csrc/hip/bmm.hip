@@ -57,7 +57,9 @@ struct Side {
   uint32_t row_origin, step_origin, row_group, step_group, rows;
   uint32_t last_run;  // first step of the last run of 8 to load: K - 8 on a plain axis, whose memory may end with the
                       // row, the last multiple of 8 below K on a blocked one, whose blocks hold whole runs
-  uint32_t last_rows, early;  // the same of the runs of 8 rows; rows by which the last tile starts early for it
+  uint32_t last_rows;  // the same of the runs of 8 rows, and what it leaves where rows of a plain axis are no multiple
+  uint32_t early;      // of 8: rows by which the last tile starts early, or, of a single tile,
+  uint32_t ragged;     // the rows in that run
   bool steps_near;    // the smaller stride is along the steps
   Axis row, step;
 };
@@ -83,6 +85,15 @@ struct BmmPlan {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+
+// The last n (1-7) of 8 elements to the front, zeros behind.
+__device__ __forceinline__ h8 tail_first(const h8& v, uint32_t n) {
+  typedef uint64_t u2 __attribute__((ext_vector_type(2)));
+  const u2 d = __builtin_bit_cast(u2, v);
+  const uint32_t cut = 16u * (8u - n);
+  return __builtin_bit_cast(
+      h8, cut < 64u ? (u2){d[0] >> cut | d[1] << (64u - cut), d[1] >> cut} : (u2){d[1] >> (cut - 64u), 0});
+}
 
 constexpr uint32_t kBmmThreads = 256;  // 4 waves, 2 x 2 over the block's tile
 
@@ -196,23 +207,26 @@ struct Stage {
         typedef uint64_t u2 __attribute__((ext_vector_type(2)));
         const uint32_t k = k0 + across() * 16u + 8u * u, c = K & 7u;  // c steps of the run across the end
         if (c && k < K && k + 8u > K) {
-          const u2 d = __builtin_bit_cast(u2, v[u]);
-          u2 r;
-          if (s.step.blk.d == 1) {  // they are the last c of the 8: to the front, zeros behind
-            const uint32_t cut = 16u * (8u - c);
-            r = cut < 64u ? (u2){d[0] >> cut | d[1] << (64u - cut), d[1] >> cut} : (u2){d[1] >> (cut - 64u), 0};
+          if (s.step.blk.d == 1) {  // they are the last c of the 8
+            v[u] = tail_first(v[u], c);
           } else {  // the first c of the 8
+            const u2 d = __builtin_bit_cast(u2, v[u]);
             const uint64_t keep = (1ull << 16u * (c & 3u)) - 1u;
-            r = c < 4u ? (u2){d[0] & keep, 0} : (u2){d[0], d[1] & keep};
+            v[u] = __builtin_bit_cast(h8, c < 4u ? (u2){d[0] & keep, 0} : (u2){d[0], d[1] & keep});
           }
-          v[u] = __builtin_bit_cast(h8, r);
         }
         if (k >= K) v[u] = zero;
       }
     }
   }
 
-  __device__ __forceinline__ void store(float* lds, const Regs& v) const {
+  __device__ __forceinline__ void store(const Side& s, float* lds, Regs& v) const {
+    if constexpr (RF) {
+      if (s.ragged && across() == s.rows / 8u) {
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) v[u] = tail_first(v[u], s.ragged);
+      }
+    }
     if (!active()) return;
     if constexpr (RF) {
 #pragma unroll
@@ -409,8 +423,8 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
       sp.trim(p.P, last * KD, K, vp[set]);
       sq.trim(p.Q, last * KD, K, vq[set]);
     }
-    sp.store(to, vp[set]);
-    sq.store(to + SP::kFloats, vq[set]);
+    sp.store(p.P, to, vp[set]);
+    sq.store(p.Q, to + SP::kFloats, vq[set]);
   };
   // chunk c = S mod PF from its buffer, chunk c + 1 into the other
   auto step = [&](auto S) __attribute__((always_inline)) {
@@ -505,8 +519,8 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     sq.trim(p.Q, 0, K, vq);
     sp.trim(p.P, 0, K, vp);
   }
-  sq.store(lds, vq);
-  sp.store(ldsp, vp);
+  sq.store(p.Q, lds, vq);
+  sp.store(p.P, ldsp, vp);
   __syncthreads();
   typename OQ::Group gq;
   oq.read(gq, lds, 0);
@@ -557,7 +571,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     // [128,400,32] x [128,32,400])
     if (more) {
       if (K < KD) sp.trim(p.P, 0, K, vp);
-      sp.store(ldsp + kTo, vp);
+      sp.store(p.P, ldsp + kTo, vp);
     }
     if (work) {
       if (p.y_vec && pt + 1u < p.ptiles) {
@@ -1223,22 +1237,19 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   // over four times as many waves
   auto blocks = [&](uint64_t r) { return (uint64_t)s.batch * ((p.P.rows + r - 1) / r) * ((p.Q.rows + r - 1) / r); };
   uint32_t w = blocks(64) >= 512 ? 2 : 1;
-  // 16-byte runs along the steps, else along the rows (rows of a plain axis
-  // may end in a partial run: the last tile then starts early, which takes a
-  // tile before it); the kernels' lane offsets are 32-bit
+  // 16-byte runs along the steps, else along the rows; the kernels' lane
+  // offsets are 32-bit
   auto steps_runs = [&](const Side& x) { return s.k >= 8 && runs_of(x.step, x.step_origin, x.step_group, 8); };
   auto rows_runs = [&](const Side& x) {
-    return runs_of(x.row, x.row_origin, x.row_group, 8) &&
-           (x.row.blk.d != 1 || x.rows % 8 == 0 || x.rows > 32u * w);
+    return runs_of(x.row, x.row_origin, x.row_group, 8) && (x.row.blk.d != 1 || x.rows >= 8);
   };
   auto near = [](const thin_desc* d) {
     int64_t extent = 0;
     for (int i = 1; i < d->rank; ++i) extent += (d->sizes[i] - 1) * d->strides[i];
     return extent < ((int64_t)1 << 30);
   };
-  auto loads = [&] { return (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)); };
-  if (w == 2 && !loads()) w = 1;  // rows that end in a partial run and fill one tile of 64, but not of 32
-  const bool fast = loads() && near(a) && near(b);
+  const bool fast =
+      (steps_runs(p.P) || rows_runs(p.P)) && (steps_runs(p.Q) || rows_runs(p.Q)) && near(a) && near(b);
   // Where b's columns come in aligned vectors, the chains on the VALU take what
   // only the gather could load (v p^T of 32 channels in blocks of 4, 1600
   // tokens: 25 us against 49) and products that leave the matrix tiles empty:
@@ -1267,7 +1278,9 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   for (Side* x : {&p.P, &p.Q}) {  // (of operands with K >= 8 steps, or with 8 or more rows, in runs)
     x->last_run = x->step.blk.d == 1 ? (uint32_t)s.k - 8u : ((uint32_t)s.k - 1u) & ~7u;
     x->last_rows = x->row.blk.d == 1 ? x->rows - 8u : (x->rows - 1u) & ~7u;
-    x->early = x->row.blk.d == 1 ? (0u - x->rows) & 7u : 0u;
+    const uint32_t part = x->row.blk.d == 1 ? x->rows & 7u : 0u;
+    if (x->rows > r) x->early = part ? 8u - part : 0u;
+    else x->ragged = part;
   }
   p.P.steps_near = unit_step(p.P.step) <= unit_step(p.P.row);
   p.Q.steps_near = unit_step(p.Q.step) <= unit_step(p.Q.row);
