@@ -364,3 +364,25 @@ def test_columns_in_vectors(gpu, batch, m, n, k):
     assert bits_equal(capi.bmm(a.to(gpu), bd), expect)
     rows = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
     assert bits_equal(capi.bmm(rows, bd), expect)
+
+
+@pytest.mark.parametrize("entries,m,k,pitch,step", [(24, 17, 8, 8, 1), (24, 17, 72, 72, 1), (24, 1, 40, 72, 1),
+                                                    (26, 1, 8, 8, 1), (24, 1, 8, 16, 2)])
+def test_more_products_than_a_launch(gpu, entries, m, k, pitch, step):
+    """A batch beyond the 2^32 threads of one launch, for each kernel: matrix
+    tiles of a short and a long reduction, chains over tiles and columns, the
+    gather.  a is a window that slides along one vector, so the sums are those
+    of a correlation, formed step by step on the device."""
+    from thintnpu_amd import capi
+    batch = (1 << entries) + 1
+    g = torch.Generator(device=gpu).manual_seed(5)
+    line = torch.randn(batch + m + step * k, generator=g, device=gpu, dtype=torch.float16)
+    a = line.as_strided((batch, m, k), (1, 1, step))
+    b = torch.randn(1, 1, pitch, generator=g, device=gpu, dtype=torch.float16)[:, :, :step * k:step]
+    acc = torch.zeros(batch + m - 1, device=gpu)
+    for i in range(k):
+        acc += line[i * step:i * step + batch + m - 1].float() * b[0, 0, i].float()
+    out = torch.full((batch, m, 1), 7.0, device=gpu, dtype=torch.float16)
+    capi.bmm(a, b.expand(batch, 1, k).transpose(1, 2), out=out)
+    expect = acc.half().view(torch.int16).unfold(0, m, 1)
+    assert torch.equal(out[:, :, 0].view(torch.int16), expect)

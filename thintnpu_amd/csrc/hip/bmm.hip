@@ -19,6 +19,8 @@
 
 #include <string.h>
 
+#include <algorithm>
+
 namespace thin {
 namespace {
 
@@ -27,7 +29,7 @@ namespace {
 struct Axis {
   FastDiv blk;
   int64_t outer, inner;
-  __device__ __forceinline__ int64_t at(uint32_t i) const {
+  __host__ __device__ __forceinline__ int64_t at(uint32_t i) const {
     const uint32_t q = blk.div(i);
     return (int64_t)q * outer + (int64_t)(i - q * blk.d) * inner;
   }
@@ -679,6 +681,12 @@ void launch_bmm(const BmmPlan& p, bool pr, bool qr, uint32_t grid, hipStream_t s
   else launch_form<SHORT, W, false, false>(p, grid, stream);
 }
 
+void launch_gather(const BmmPlan& p, uint32_t rp, uint32_t grid, hipStream_t stream) {
+  if (rp == 64) hipLaunchKernelGGL((bmm_gather_kernel<64, 16>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else if (rp == 16) hipLaunchKernelGGL((bmm_gather_kernel<16, 64>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else hipLaunchKernelGGL((bmm_gather_kernel<32, 32>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+}
+
 // ---------------------------------------------------------------- chains on the VALU
 // A chain of fmas per output, a lane to an output column, for products that
 // leave the matrix tiles mostly empty (few rows of a, short reductions, many
@@ -1075,13 +1083,33 @@ thin_status check_out(const thin_desc* out, const BmmShape& s, const thin_bmm_la
 }
 
 template <int RM>
-void launch_stream(const ChainPlan& p, uint32_t grid, hipStream_t stream) {
+void launch_stream_rows(const ChainPlan& p, uint32_t grid, hipStream_t stream) {
   if (p.k <= 32)
     hipLaunchKernelGGL((chain_stream_kernel<RM, 1, 4>), dim3(grid), dim3(64), 0, stream, p);
   else if (p.k <= 64)
     hipLaunchKernelGGL((chain_stream_kernel<RM, 1, 8>), dim3(grid), dim3(64), 0, stream, p);
   else
     hipLaunchKernelGGL((chain_stream_kernel<RM, 8, 8>), dim3(grid), dim3(64), 0, stream, p);
+}
+
+void launch_stream(const ChainPlan& p, int rm, uint32_t grid, hipStream_t stream) {
+  if (rm == 4) launch_stream_rows<4>(p, grid, stream);
+  else if (rm == 2) launch_stream_rows<2>(p, grid, stream);
+  else launch_stream_rows<1>(p, grid, stream);
+}
+
+void launch_tile(const ChainPlan& p, int rm, uint32_t grid, hipStream_t stream) {
+  if (rm == 4) hipLaunchKernelGGL(chain_tile_kernel<4>, dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else if (rm == 2) hipLaunchKernelGGL(chain_tile_kernel<2>, dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  else hipLaunchKernelGGL(chain_tile_kernel<1>, dim3(grid), dim3(kBmmThreads), 0, stream, p);
+}
+
+// Entries of the batch that one launch takes: a launch holds fewer than 2^32
+// threads (it wraps beyond, without an error), and parts in multiples of 16
+// begin at whole channel blocks of a grouped output.  0: not even 16 fit.
+int64_t batch_part(int64_t batch, uint64_t blocks, uint32_t threads) {
+  const int64_t most = (int64_t)(UINT32_MAX / threads / blocks);
+  return most >= batch ? batch : most & ~(int64_t)15;
 }
 
 // The product as chains; a and b as in thin_layout_bmm, b streamable and of
@@ -1106,37 +1134,31 @@ thin_status launch_chains(const Mat& a, const Mat& b, int64_t b_extent, const Bm
   p.b_bytes = (uint32_t)(b_extent * 2);
   p.b_vrun = b.row.blk.d == 1 ? 0u : b.row.blk.d / 8u;
   p.b_vjump = b.row.blk.d == 1 ? 0u : (uint32_t)((b.row.outer - b.row.blk.d) * 2);
-  auto tiles = [&](int rows) { return (uint64_t)s.batch * ((s.m + rows - 1) / rows) * p.ntiles; };
-  if (p.k % 8 == 0 && b.col.blk.d == 1 && b.col.outer >= 64) {
-    // the tallest tile that leaves every SIMD about a wave
-    const int rm = tiles(16) * 4 >= 1024 ? 4 : tiles(8) * 4 >= 1024 ? 2 : 1;
-    p.mtiles = (uint32_t)((s.m + 4 * rm - 1) / (4 * rm));
-    const uint64_t grid = tiles(4 * rm);
-    THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
-    if (rm == 4)
-      hipLaunchKernelGGL(chain_tile_kernel<4>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-    else if (rm == 2)
-      hipLaunchKernelGGL(chain_tile_kernel<2>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-    else
-      hipLaunchKernelGGL(chain_tile_kernel<1>, dim3((uint32_t)grid), dim3(kBmmThreads), 0, stream, p);
-    THIN_LAUNCH_CHECK("chain_tile_kernel");
-    return THIN_OK;
-  }
-  // rows per wave: 2; 1 when that leaves under half a wave per SIMD, 4 when it
-  // would queue more than 8 waves per SIMD
-  const int rm = tiles(2) < 512 ? 1 : tiles(2) > 8192 ? 4 : 2;
-  p.mtiles = (uint32_t)((s.m + rm - 1) / rm);
+  const bool tile = p.k % 8 == 0 && b.col.blk.d == 1 && b.col.outer >= 64;
+  const int unit = tile ? 4 : 1;  // rows of a block for RM = 1
+  auto tiles = [&](int rm) { return (uint64_t)((s.m + unit * rm - 1) / (unit * rm)) * p.ntiles; };  // of one entry
+  auto waves = [&](int rm) { return (uint64_t)s.batch * tiles(rm) * (uint64_t)unit; };
+  // tile: the tallest that leaves every SIMD about a wave.  Stream: two rows a
+  // wave; one when that leaves under half a wave per SIMD, four when it would
+  // queue more than 8 waves per SIMD
+  const int rm = tile ? (waves(4) >= 1024 ? 4 : waves(2) >= 1024 ? 2 : 1) : waves(2) < 512 ? 1 : waves(2) > 8192 ? 4 : 2;
+  p.mtiles = (uint32_t)(tiles(rm) / p.ntiles);
   p.div_mt = FastDiv::make(p.mtiles);
   p.div_nt = FastDiv::make(p.ntiles);
-  const uint64_t grid = tiles(rm);
-  THIN_REQUIRE(grid < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
-  if (rm == 4)
-    launch_stream<4>(p, (uint32_t)grid, stream);
-  else if (rm == 2)
-    launch_stream<2>(p, (uint32_t)grid, stream);
-  else
-    launch_stream<1>(p, (uint32_t)grid, stream);
-  THIN_LAUNCH_CHECK("chain_stream_kernel");
+  const int64_t part = batch_part(s.batch, tiles(rm), tile ? kBmmThreads : 64u);
+  THIN_REQUIRE(part > 0, THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
+  for (int64_t b0 = 0; b0 < s.batch; b0 += part) {
+    const uint32_t grid = (uint32_t)(std::min(part, s.batch - b0) * (int64_t)tiles(rm));
+    if (tile) launch_tile(p, rm, grid, stream);
+    else launch_stream(p, rm, grid, stream);
+    THIN_LAUNCH_CHECK("chain_kernel");
+    for (Mat* x : {&p.a, &p.b, &p.y}) {
+      x->p += part * x->batch;
+      x->row_origin += (uint32_t)part * x->row_group;
+      x->col_origin += (uint32_t)part * x->col_group;
+    }
+    p.b_bytes -= (uint32_t)(part * b.batch * 2);
+  }
   return THIN_OK;
 }
 
@@ -1268,8 +1290,7 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   };
   int64_t b_extent = 1;  // elements from b's data pointer to its last element, + 1
   for (int d = 0; d < b->rank; ++d) b_extent += (b->sizes[d] - 1) * b->strides[d];
-  // (a launch holds 2^32 threads: 2^24 blocks of the matrix kernels)
-  if (streamable_b(bm) && b_extent * 2 < ((int64_t)1 << 31) && (!fast || sparse() || tiles >= ((uint64_t)1 << 24)))
+  if (streamable_b(bm) && b_extent * 2 < ((int64_t)1 << 31) && (!fast || sparse()))
     return launch_chains(am, bm, b_extent, s, out, layout, stream);
   if (!fast) w = 1;
   const bool one = s.k <= 32;  // one chunk of steps
@@ -1288,7 +1309,6 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
   p.ptiles = (p.P.rows + rp - 1) / rp;
   p.qtiles = FastDiv::make((p.Q.rows + rq - 1) / rq);
   p.y_vec = runs_of(p.yp, 0, p.yp_group, 4 * w) ? 1u : 0u;
-  THIN_REQUIRE(blocks(r) < ((uint64_t)1 << 31), THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
   p.span = 1;
   if (fast && one) {
     // as many P tiles a block as leave a block or two a compute unit, in even
@@ -1309,22 +1329,25 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
     p.Q.hop = (int64_t)(kd / p.Q.step.blk.d) * p.Q.step.outer * 2;
   }
   p.pblocks = FastDiv::make((p.ptiles + p.span - 1) / p.span);
-  const uint32_t grid = (uint32_t)((uint64_t)s.batch * p.qtiles.d * p.pblocks.d);
-  if (!fast && rp == 64)
-    hipLaunchKernelGGL((bmm_gather_kernel<64, 16>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
-  else if (!fast && rp == 16)
-    hipLaunchKernelGGL((bmm_gather_kernel<16, 64>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
-  else if (!fast)
-    hipLaunchKernelGGL((bmm_gather_kernel<32, 32>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
-  else if (one && w == 2)
-    launch_bmm<true, 2>(p, pr, qr, grid, stream);
-  else if (one)
-    launch_bmm<true, 1>(p, pr, qr, grid, stream);
-  else if (w == 2)
-    launch_bmm<false, 2>(p, pr, qr, grid, stream);
-  else
-    launch_bmm<false, 1>(p, pr, qr, grid, stream);
-  THIN_LAUNCH_CHECK("bmm_kernel");
+  const uint64_t per = (uint64_t)p.qtiles.d * p.pblocks.d;  // blocks of an entry
+  const int64_t part = batch_part(s.batch, per, kBmmThreads);
+  THIN_REQUIRE(part > 0, THIN_ERR_UNSUPPORTED, "bmm: too many output tiles");
+  for (int64_t b0 = 0; b0 < s.batch; b0 += part) {
+    const uint32_t grid = (uint32_t)(std::min(part, s.batch - b0) * (int64_t)per);
+    if (!fast) launch_gather(p, rp, grid, stream);
+    else if (one && w == 2) launch_bmm<true, 2>(p, pr, qr, grid, stream);
+    else if (one) launch_bmm<true, 1>(p, pr, qr, grid, stream);
+    else if (w == 2) launch_bmm<false, 2>(p, pr, qr, grid, stream);
+    else launch_bmm<false, 1>(p, pr, qr, grid, stream);
+    THIN_LAUNCH_CHECK("bmm_kernel");
+    for (Side* x : {&p.P, &p.Q}) {
+      x->p += part * x->batch;
+      x->row_origin += (uint32_t)part * x->row_group;
+      x->step_origin += (uint32_t)part * x->step_group;
+    }
+    p.y += part * p.ybatch;
+    if (p.yp_group && b0 + part < s.batch) p.y += p.yp.at((uint32_t)part * p.yp_group);
+  }
   return THIN_OK;
 }
 
