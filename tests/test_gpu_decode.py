@@ -192,3 +192,23 @@ def test_decode_row_ends(gpu, a, nc):
     capi.detect_decode(boxes.to(gpu), head[:, :, 1:1 + a], shapes, strides, out=wide[:, :, 3:3 + a])
     assert bits_equal(wide[:, :, 3:3 + a].cpu(), want.cpu())
     assert wide[:, :, :3].eq(7).all() and wide[:, :, 3 + a:].eq(7).all()
+
+
+@pytest.mark.parametrize("batch,nc,a", [(6, 11200, 9), (4, 11600, 13), (3, 13400, 15), (2, 13100, 23),
+                                        (4, 80, 2050), (3, 70, 4101), (8, 70, 4101), (5, 186, 2795)])
+def test_decode_row_ends_in_vectors(gpu, batch, nc, a):
+    """The same with enough class scores for 16-byte units at any alignment,
+    one unit a thread and more, the last two with outputs of 4 MiB and more
+    (streaming loads and stores): into a tensor, and into a view at an odd
+    offset whose surroundings stay as they were."""
+    from thintnpu_amd import capi
+    shapes, strides = [(1, a - 2), (1, 2)], [8.0, 16.0]
+    boxes, scores = inputs(batch, nc, shapes, a)
+    want = composed(capi, gpu, boxes, scores, shapes, strides, False)
+    assert bits_equal(capi.detect_decode(boxes.to(gpu), scores.to(gpu), shapes, strides).cpu(), want.cpu())
+    wide = torch.full((batch, 4 + nc, a + 5), 7.0, dtype=torch.float16, device=gpu)
+    head = torch.zeros((batch, nc, a + 3), dtype=torch.float16, device=gpu)
+    head[:, :, 1:1 + a] = scores.to(gpu)
+    capi.detect_decode(boxes.to(gpu), head[:, :, 1:1 + a], shapes, strides, out=wide[:, :, 3:3 + a])
+    assert bits_equal(wide[:, :, 3:3 + a].cpu(), want.cpu())
+    assert wide[:, :, :3].eq(7).all() and wide[:, :, 3 + a:].eq(7).all()

@@ -666,9 +666,14 @@ __global__ __launch_bounds__(kThreads) void dfl_expect_rows_kernel(DflPlan p) {
 // Blocks [0, box_blocks) decode boxes: a thread takes one axis (x or y) of V
 // adjacent anchors and so the box sides axis and axis+2.  The remaining blocks
 // apply the sigmoid to the class logits, 8 adjacent ones at a time.  The bound
-// is HBM; at one logit a thread, which only rows of scattered anchors or fewer
-// than 8 still take, it is the issue of 2-byte accesses instead.
+// is HBM; at one logit a thread (scattered anchors, fewer than 8 of them, or
+// few unaligned rows) it is the issue of 2-byte accesses instead.
 constexpr int kMaxLevels = 8;
+// Class scores from which rows of any alignment are worth the vector form: it
+// has eight sigmoids and a row end a thread one after another.  [1,80,4101]
+// 3.32 us against 3.12 an element a thread, [3,80,2100] 3.50 / 3.34,
+// [1,80,8400] at an odd offset 3.28 / 3.48, [3,80,4101] 3.53 / 3.94.
+constexpr int64_t kEndsScores = 600000;
 
 struct DecodePlan {
   const _Float16* boxes;  // [B,64,A] DFL logits, or [B,4,A] distances (direct)
@@ -824,20 +829,22 @@ __global__ __launch_bounds__(kThreads) void detect_decode_kernel(DecodePlan p) {
     vec x[SU];
 #pragma unroll
     for (uint32_t s = 0; s < SU; ++s) {
-      // a partial unit loads the row's last 8 instead, unused
+      // a partial unit loads the row's last 8, of which it owns the last `left`
       const vec* src = reinterpret_cast<const vec*>(ENDS ? sp[s] - (8u - min(left[s], 8u)) : sp[s]);
       x[s] = LOAD == 2 ? __builtin_nontemporal_load(src) : *src;
     }
 #pragma unroll
     for (uint32_t s = 0; s < SU; ++s) {
       if (v0 + s * kThreads >= p.score_units) break;
-      if (ENDS && left[s] < 8u) {
-        for (uint32_t j = 0; j < left[s]; ++j) op[s][j] = (_Float16)dev::sigmoid_fast((float)sp[s][j]);
-        continue;
-      }
       vec y;
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = (_Float16)dev::sigmoid_fast((float)x[s][j]);
+      if (ENDS && left[s] < 8u) {
+#pragma unroll
+        for (uint32_t j = 1; j < 8; ++j)
+          if (j >= 8u - left[s]) op[s][(int32_t)(j + left[s]) - 8] = y[j];
+        continue;
+      }
       if constexpr (LOAD == 2) __builtin_nontemporal_store(y, reinterpret_cast<vec*>(op[s]));
       else *reinterpret_cast<vec*>(op[s]) = y;
     }
@@ -1187,9 +1194,9 @@ extern "C" thin_status thin_detect_decode(const thin_desc* boxes, const thin_des
   p.direct = boxes->sizes[1] == 4 ? 1 : 0;
   const bool vb = A % 2 == 0 && p.ba == 1 && p.oa == 1 && aligned(boxes->data, 4) && aligned(out->data, 4) &&
                   p.bb % 2 == 0 && p.bc % 2 == 0 && p.ob % 2 == 0 && p.oc % 2 == 0;
-  const bool vs = A >= 8 && p.sa == 1 && p.oa == 1;
   const bool ends = !(A % 8 == 0 && aligned(scores->data, 16) && aligned(out->data, 16) && p.sb % 8 == 0 &&
                       p.sc % 8 == 0 && p.ob % 8 == 0 && p.oc % 8 == 0);
+  const bool vs = A >= 8 && p.sa == 1 && p.oa == 1 && (!ends || (int64_t)B * nc * A >= kEndsScores);
   const int VB = vb ? 2 : 1, VS = vs ? 8 : 1;
   p.apairs = (uint32_t)(A / VB);
   const uint64_t box_units = (uint64_t)B * 2 * p.apairs;
