@@ -1302,6 +1302,7 @@ struct RunsPlan {
   uint32_t A, nc, K;
   uint32_t runs;          // runs per image: ceil(A / kRun)
   uint32_t q, m, m2;      // finish: prefix length and ranks of the candidate bounds (host: A and K only)
+  uint32_t q_last;        // the prefix length in the last run
   uint32_t rows_per;      // finish: stage-1 ranks per gather pass, kFinishThreads / nc
   int32_t agnostic;
   int32_t vec_classes;    // anchors contiguous in aligned 16-byte groups
@@ -1859,7 +1860,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   const u4v* recs = reinterpret_cast<const u4v*>(p.runs_rec + (size_t)b * nl * kRun);
   const u2v* sides = reinterpret_cast<const u2v*>(p.runs_side + (size_t)b * nl * kRun);
   const uint32_t k8 = tid & 7u;
-  const uint32_t qrec = p.runs_rec[((size_t)b * nl + min(tid, nl - 1u)) * kRun + p.q - 1u];
+  const uint32_t qrec = p.runs_rec[((size_t)b * nl + min(tid, nl - 1u)) * kRun + (tid + 1u < nl ? p.q : p.q_last) - 1u];
   u4v held[4];
   u2v held_side[4];
   auto run_of = [&](uint32_t i) { return WIDE ? i * kHeldRuns + (tid >> 3) : tid >> 3; };
@@ -1875,7 +1876,6 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
     count2 = 0;
     nx = 0;
     nxr = 0;
-    if (p.m == 0) bound[0] = bound[1] = kPad - 1u;  // no such rank: every record
   }
   __syncthreads();
 
@@ -2256,7 +2256,7 @@ SplitShape split_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnosti
 // scores beyond its LDS table).
 struct RunsShape {
   bool ok;
-  uint32_t runs, q, m, m2, rows_per;
+  uint32_t runs, q, q_last, m, m2, rows_per;
 };
 
 RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic, int64_t image_extent, bool wide) {
@@ -2268,21 +2268,20 @@ RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic,
   if (!agnostic && (nc > (int64_t)kFinishThreads || K * nc > (int64_t)kPairTable)) return r;
   r.runs = (uint32_t)((A + kRun - 1) / kRun);
   // The bounds' prefix length q and rank m: m * q >= K over the runs of q or
-  // more records, at three quarters of them or, where K is most of A, as low
-  // as they allow (none: m = 0, every record).  m2: the rank up to which
-  // runs would have q records if each held a Poisson count of 1.25 K / runs.
+  // more records, the first q with m at three quarters of those runs, else the
+  // first with m among them.  m2: the rank up to which runs would have q
+  // records if each held a Poisson count of 1.25 K / runs.
   const int64_t last = A - (int64_t)(r.runs - 1) * kRun;
   for (uint32_t q = 1; q <= kRun; ++q) {
     const int64_t have = (int64_t)r.runs - (last < (int64_t)q ? 1 : 0), m = (K + q - 1) / q;
-    if (m > have) continue;
-    r.q = q;
-    r.m = (uint32_t)m;
-    if (4 * m > 3 * have) continue;
-    break;
+    const bool low = 4 * m <= 3 * have;
+    if (low || (m <= have && !r.m)) {
+      r.q = r.q_last = q;
+      r.m = (uint32_t)m;
+    }
+    if (low) break;
   }
-  if (!r.m) {
-    r.q = 1;
-  } else {
+  if (r.m) {
     const double mean = 1.25 * (double)K / r.runs;
     double term = exp(-mean), below = 0;
     for (uint32_t i = 0; i < r.q; ++i) {
@@ -2291,6 +2290,14 @@ RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic,
     }
     const double rank = (1.0 - below) * r.runs;
     r.m2 = rank < 1 ? 1 : rank > r.m ? r.m : (uint32_t)rank;
+  } else {
+    // K is most of A: the smallest prefix length at which all prefixes, the
+    // last run's as long as it is, hold K records; the bound is the largest of
+    // their ends
+    const int64_t q = (K + r.runs - 1) / r.runs;
+    r.q = (uint32_t)(q <= last ? q : (K - last + r.runs - 2) / (r.runs - 1));
+    r.q_last = (uint32_t)std::min((int64_t)r.q, last);
+    r.m = r.m2 = r.runs;
   }
   r.rows_per = agnostic ? 0u : (uint32_t)(kFinishThreads / nc);
   r.ok = true;
@@ -2452,6 +2459,7 @@ thin_status select_run(const thin_desc* decoded, int64_t max_det, bool agn, void
     rp.K = (uint32_t)K;
     rp.runs = w.two.runs;
     rp.q = w.two.q;
+    rp.q_last = w.two.q_last;
     rp.m = w.two.m;
     rp.m2 = w.two.m2;
     rp.rows_per = w.two.rows_per;
