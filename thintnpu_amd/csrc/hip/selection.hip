@@ -1854,8 +1854,9 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   const u4v* info_g = p.info + (size_t)b * p.A;
 
   // the q-th record of every run and the threads' records, with their row
-  // keys: every load issued before any is used (runs past the last one read
-  // it again, unused)
+  // keys: every load issued before any is used (runs past the last one read it
+  // again, unused; waves with none but those load nothing, which an image of a
+  // few runs would wait for: 0.5 us of 11 at 1000 anchors)
   typedef uint32_t u2v __attribute__((ext_vector_type(2)));
   const u4v* recs = reinterpret_cast<const u4v*>(p.runs_rec + (size_t)b * nl * kRun);
   const u2v* sides = reinterpret_cast<const u2v*>(p.runs_side + (size_t)b * nl * kRun);
@@ -1864,11 +1865,13 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   u4v held[4];
   u2v held_side[4];
   auto run_of = [&](uint32_t i) { return WIDE ? i * kHeldRuns + (tid >> 3) : tid >> 3; };
+  if (WIDE || (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)) * 8u < nl) {
 #pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t at = min(run_of(i), nl - 1u) * (kRun / 4) + (WIDE ? 0u : i * 8u) + k8;
-    held[i] = recs[at];
-    held_side[i] = sides[at];
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t at = min(run_of(i), nl - 1u) * (kRun / 4) + (WIDE ? 0u : i * 8u) + k8;
+      held[i] = recs[at];
+      held_side[i] = sides[at];
+    }
   }
   if (tid < kRuns) qth[tid] = tid < nl ? qrec : kPad;
   if (tid == 0) {
