@@ -188,8 +188,8 @@ def test_selection_graph_replays(gpu, noalloc):
 
 def _scores_case(kind, batch, anchors, nc, seed):
     """Independent scores; all the best ones within a few hundred neighbouring
-    anchors (more candidates in a run than are held of a long image); or eight
-    score levels (thousands of ties)."""
+    anchors (more candidates in a run than are held of a long image); eight
+    score levels (thousands of ties); or zero but for a few anchors."""
     g = torch.Generator().manual_seed(seed)
     s = torch.rand(batch, anchors, nc, generator=g)
     if kind == "clustered":
@@ -198,17 +198,20 @@ def _scores_case(kind, batch, anchors, nc, seed):
         s[:, first:first + 450] += 0.5
     elif kind == "tied":
         s = (s * 8).floor() / 8
+    elif kind == "thresholded":
+        s = s * (torch.rand(batch, anchors, 1, generator=g) * anchors < 40)
     boxes = torch.randn(batch, anchors, 4, generator=g)
     return torch.cat((boxes, s), -1).half()
 
 
-@pytest.mark.parametrize("kind", ["independent", "clustered", "tied"])
+@pytest.mark.parametrize("kind", ["independent", "clustered", "tied", "thresholded"])
 @pytest.mark.parametrize("batch,anchors,nc,max_det,layout", [
     (1, 16385, 6, 300, "transposed"),   # first size past the runs held whole, scalar loads
     (2, 33600, 8, 300, "transposed"),   # 1280 x 1280 pixels; 526 runs: 128 threads each
     (1, 33600, 8, 300, "contiguous"),
     (1, 65536, 5, 1024, "transposed"),  # the most anchors and records
     (1, 65537, 5, 300, "transposed"),   # one more: the one-workgroup path
+    (1, 33600, 40, 300, "transposed"),  # ties in most of the pairs as well
     (9, 8400, 12, 300, "transposed"),   # many runs of images held whole
     (4, 16384, 7, 1000, "transposed"),
     (1, 130, 4, 130, "transposed"),     # K the whole image: no rank bounds it

@@ -1303,6 +1303,7 @@ struct RunsPlan {
   uint32_t runs;          // runs per image: ceil(A / kRun)
   uint32_t q, m, m2;      // finish: prefix length and ranks of the candidate bounds (host: A and K only)
   uint32_t q_last;        // the prefix length in the last run
+  uint32_t ends;          // whole runs that hold K records, 0: not that many runs
   uint32_t rows_per;      // finish: stage-1 ranks per gather pass, kFinishThreads / nc
   int32_t agnostic;
   int32_t vec_classes;    // anchors contiguous in aligned 16-byte groups
@@ -1887,76 +1888,88 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
     v += dev::lane_xor_bits<2>(v);
     return v + dev::lane_xor_bits<4>(v);
   };
-  // the ranks of the q-th records among themselves (records are unique; runs
-  // shorter than q hold kPad there and come last)
+  // Where more candidates are left than one sort holds (a key that thousands
+  // of anchors share, or the best anchors all in a few runs), a second pass
+  // takes the ends of whole runs as the records to rank: 300 tied anchors then
+  // leave 384.
+  for (bool ends = false;; ends = true) {
+    const uint32_t m = ends ? p.ends : p.m, m2 = ends ? p.ends : p.m2;
+    // the ranks of the q-th records among themselves (records are unique; runs
+    // shorter than q hold kPad there and come last)
 #pragma unroll
-  for (uint32_t i = 0; i < (WIDE ? 4u : 1u); ++i) {
-    const uint32_t l = run_of(i), mine = qth[l];
-    uint32_t below = 0;
-    for (uint32_t j = k8; j * 4u < nl; j += 8) {
-      const u4v w = reinterpret_cast<const u4v*>(qth)[j];
-      below += (w.x < mine) + (w.y < mine) + (w.z < mine) + (w.w < mine);
-    }
-    below = sum8(below);
-    if (k8 == 0 && l < nl && mine != kPad) {
-      if (below + 1u == p.m) bound[0] = mine;
-      if (below + 1u == p.m2) bound[1] = mine;
-    }
-  }
-  __syncthreads();
-  const uint32_t R0 = bound[0], R1 = bound[1];
-  {
-    uint32_t c0 = 0, c1 = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const u4v w = held[i];
-      c0 += (w.x <= R0) + (w.y <= R0) + (w.z <= R0) + (w.w <= R0);
-      c1 += (w.x <= R1) + (w.y <= R1) + (w.z <= R1) + (w.w <= R1);
-      if (WIDE || i == 3) {
-        const uint32_t l = run_of(i);
-        c0 = sum8(c0);
-        c1 = sum8(c1);
-        if (WIDE) {
-          for (uint32_t t = 1; t < 4 && c0 == 32u * t; ++t) {
-            const u4v x = recs[min(l, nl - 1u) * (kRun / 4) + t * 8u + k8];
-            c0 += sum8((x.x <= R0) + (x.y <= R0) + (x.z <= R0) + (x.w <= R0));
-            c1 += sum8((x.x <= R1) + (x.y <= R1) + (x.z <= R1) + (x.w <= R1));
-          }
-        }
-        if (k8 == 0) {
-          cnt[l] = l < nl ? c0 : 0u;
-          cnt2[l] = l < nl ? c1 : 0u;
-        }
-        c0 = 0;
-        c1 = 0;
+    for (uint32_t i = 0; i < (WIDE ? 4u : 1u); ++i) {
+      const uint32_t l = run_of(i), mine = qth[l];
+      uint32_t below = 0;
+      for (uint32_t j = k8; j * 4u < nl; j += 8) {
+        const u4v w = reinterpret_cast<const u4v*>(qth)[j];
+        below += (w.x < mine) + (w.y < mine) + (w.z < mine) + (w.w < mine);
+      }
+      below = sum8(below);
+      if (k8 == 0 && l < nl && mine != kPad) {
+        if (below + 1u == m) bound[0] = mine;
+        if (below + 1u == m2) bound[1] = mine;
       }
     }
-  }
-  __syncthreads();
-  if (tid < 64) {
-    constexpr uint32_t kPer = kRuns / 64;
-    uint32_t s0 = 0, s1 = 0;
+    __syncthreads();
+    // (a second pass: the lower of the bounds, twice)
+    const uint32_t R0 = ends ? min(bound[0], chosen) : bound[0], R1 = ends ? R0 : bound[1];
+    {
+      uint32_t c0 = 0, c1 = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-      s0 += cnt[tid * kPer + j];
-      s1 += cnt2[tid * kPer + j];
+      for (uint32_t i = 0; i < 4; ++i) {
+        const u4v w = held[i];
+        c0 += (w.x <= R0) + (w.y <= R0) + (w.z <= R0) + (w.w <= R0);
+        c1 += (w.x <= R1) + (w.y <= R1) + (w.z <= R1) + (w.w <= R1);
+        if (WIDE || i == 3) {
+          const uint32_t l = run_of(i);
+          c0 = sum8(c0);
+          c1 = sum8(c1);
+          if (WIDE) {
+            for (uint32_t t = 1; t < 4 && c0 == 32u * t; ++t) {
+              const u4v x = recs[min(l, nl - 1u) * (kRun / 4) + t * 8u + k8];
+              c0 += sum8((x.x <= R0) + (x.y <= R0) + (x.z <= R0) + (x.w <= R0));
+              c1 += sum8((x.x <= R1) + (x.y <= R1) + (x.z <= R1) + (x.w <= R1));
+            }
+          }
+          if (k8 == 0) {
+            cnt[l] = l < nl ? c0 : 0u;
+            cnt2[l] = l < nl ? c1 : 0u;
+          }
+          c0 = 0;
+          c1 = 0;
+        }
+      }
     }
-    const uint32_t i0 = wave_scan_u32(s0), i1 = wave_scan_u32(s1);
-    const bool low = (uint32_t)__builtin_amdgcn_readlane((int)i1, 63) >= K;
-    uint32_t at = low ? i1 - s1 : i0 - s0;
+    __syncthreads();
+    if (tid < 64) {
+      constexpr uint32_t kPer = kRuns / 64;
+      uint32_t s0 = 0, s1 = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-      const uint32_t l = tid * kPer + j, n = low ? cnt2[l] : cnt[l];
-      off[l] = at;
-      cnt[l] = n;
-      at += n;
+      for (uint32_t j = 0; j < kPer; ++j) {
+        s0 += cnt[tid * kPer + j];
+        s1 += cnt2[tid * kPer + j];
+      }
+      const uint32_t i0 = wave_scan_u32(s0), i1 = wave_scan_u32(s1);
+      const bool low = (uint32_t)__builtin_amdgcn_readlane((int)i1, 63) >= K;
+      uint32_t at = low ? i1 - s1 : i0 - s0;
+#pragma unroll
+      for (uint32_t j = 0; j < kPer; ++j) {
+        const uint32_t l = tid * kPer + j, n = low ? cnt2[l] : cnt[l];
+        off[l] = at;
+        cnt[l] = n;
+        at += n;
+      }
+      if (tid == 63) {
+        total = at;
+        chosen = low ? R1 : R0;
+      }
     }
-    if (tid == 63) {
-      total = at;
-      chosen = low ? R1 : R0;
-    }
+    __syncthreads();
+    if (ends || total <= kSortCap || !p.ends) break;
+    const uint32_t end = p.runs_rec[((size_t)b * nl + min(tid, nl - 1u)) * kRun + kRun - 1u];
+    if (tid < kRuns) qth[tid] = tid < nl ? end : kPad;
+    __syncthreads();
   }
-  __syncthreads();
   const uint32_t C = total, Rkey = chosen >> 16;
   // each thread's candidates: record, row key, position
   auto candidates = [&](auto&& f) {
@@ -2030,7 +2043,7 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   block_sort(sortbuf, n1, xch);
 
   if (few) {
-      if (tid < C) info_slot[tid] = my_info;
+    if (tid < C) info_slot[tid] = my_info;
     if (fast && grow < G) {
 #pragma unroll
       for (uint32_t i = 0; i < kXBatch; ++i) {
@@ -2178,25 +2191,55 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
     }
   }
   __syncthreads();
-  // the survivors sorted, or (more than kSortCap: ties) the K-th smallest pair
-  // record selected over the whole table and the K records up to it sorted
+  // the survivors sorted, or (more than kSortCap: ties) K of them: the pairs
+  // below T1 and the first of those at T1 by pair index, or, where the pairs
+  // below T1 are more than K, the records up to the K-th smallest
   const uint32_t S = count;
   uint32_t have2 = K;
   if (S <= kSortCap) {
     have2 = S;
   } else {
-    const uint32_t total = K * nc;
-    if (tid == 0) count2 = 0;
-    const uint32_t T = radix_select(
-        [&](auto&& f) {
-          for (uint32_t i = tid; i < total; i += kFinishThreads) f((run_key(table[i]) << 16) | i);
-        },
-        K, hist, sel);
-    for (uint32_t i = tid; i < total; i += kFinishThreads) {
-      const uint32_t rec = (run_key(table[i]) << 16) | i;
-      if (rec <= T) {
-        const uint32_t slot = atomicAdd(&count2, 1u);
-        if (slot < kSortCap) s2buf[slot] = rec;  // exactly K
+    const uint32_t pairs = K * nc, lane = tid & 63u, wave = tid >> 6;
+    __syncthreads();  // S is read
+    if (tid == 0) count = count2 = 0;
+    __syncthreads();
+    uint32_t less = 0;
+    for (uint32_t i = tid; i < pairs; i += kFinishThreads) less += run_key(table[i]) < T1;
+    if (less) atomicAdd(&count, less);
+    __syncthreads();
+    const uint32_t L = count;
+    // the pairs at most `top` into the slots from 0 on (at most K of them)
+    auto take = [&](uint32_t top) {
+      for (uint32_t i = tid; i < pairs; i += kFinishThreads) {
+        const uint32_t rec = (run_key(table[i]) << 16) | i;
+        if (rec <= top) {
+          const uint32_t slot = atomicAdd(&count2, 1u);
+          if (slot < kSortCap) s2buf[slot] = rec;
+        }
+      }
+    };
+    if (L > K) {
+      take(radix_select(
+          [&](auto&& f) {
+            for (uint32_t i = tid; i < pairs; i += kFinishThreads) f((run_key(table[i]) << 16) | i);
+          },
+          K, hist, sel));
+    } else {
+      if (L) take((T1 << 16) - 1u);
+      for (uint32_t base = 0, at = L; at < K && base < pairs; base += kFinishThreads) {
+        const uint32_t i = base + tid;
+        const uint64_t tied = __ballot(i < pairs && run_key(table[i]) == T1);
+        if (lane == 0) hist[wave] = (uint32_t)__popcll(tied);
+        __syncthreads();
+        uint32_t slot = at + (uint32_t)__popcll(tied & ((1ull << lane) - 1u)), found = 0;
+        for (uint32_t w = 0; w < kFinishThreads / 64; ++w) {
+          const uint32_t n = hist[w];
+          if (w < wave) slot += n;
+          found += n;
+        }
+        if ((tied >> lane & 1u) && slot < K) s2buf[slot] = (T1 << 16) | i;
+        at += found;
+        __syncthreads();
       }
     }
   }
@@ -2259,7 +2302,7 @@ SplitShape split_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnosti
 // scores beyond its LDS table).
 struct RunsShape {
   bool ok;
-  uint32_t runs, q, q_last, m, m2, rows_per;
+  uint32_t runs, q, q_last, m, m2, ends, rows_per;
 };
 
 RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic, int64_t image_extent, bool wide) {
@@ -2302,6 +2345,8 @@ RunsShape runs_shape(int64_t B, int64_t A, int64_t nc, int64_t K, bool agnostic,
     r.q_last = (uint32_t)std::min((int64_t)r.q, last);
     r.m = r.m2 = r.runs;
   }
+  const uint32_t ends = (uint32_t)((K + kRun - 1) / kRun);
+  if (ends <= (uint32_t)(A / kRun)) r.ends = ends;
   r.rows_per = agnostic ? 0u : (uint32_t)(kFinishThreads / nc);
   r.ok = true;
   return r;
@@ -2463,6 +2508,7 @@ thin_status select_run(const thin_desc* decoded, int64_t max_det, bool agn, void
     rp.runs = w.two.runs;
     rp.q = w.two.q;
     rp.q_last = w.two.q_last;
+    rp.ends = w.two.ends;
     rp.m = w.two.m;
     rp.m2 = w.two.m2;
     rp.rows_per = w.two.rows_per;
