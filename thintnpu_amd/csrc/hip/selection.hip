@@ -1307,7 +1307,7 @@ struct RunsPlan {
   uint32_t rows_per;      // finish: stage-1 ranks per gather pass, kFinishThreads / nc
   int32_t agnostic;
   int32_t vec_classes;    // anchors contiguous in aligned 16-byte groups
-  int32_t row_classes;    // classes contiguous, rows in aligned 8-byte chunks, nc % 4 == 0
+  int32_t row_classes;    // classes contiguous, four of them or more
   uint32_t* runs_rec;     // [B, runs, kRun]: sorted records
   uint16_t* runs_side;    // [B, runs, kRun]: row key of each record's anchor
   u4v* info;              // [B, A] halves: box[4], class-max bits, class, second key, second class
@@ -1673,22 +1673,28 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
   } else if constexpr (kMany) {
   } else if (p.row_classes) {
     // four lanes per anchor: lane g reads the anchor's 8-byte class chunks g,
-    // g + 4, ... (lane 0 also the box chunk before them), then the quad merges
-    // its four triples in two exchanges, leaving the anchor's three in every lane
-    typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+    // g + 4, ... (lane 0 also the box chunk before them), at any alignment, then
+    // the quad merges its four triples in two exchanges, leaving the anchor's
+    // three in every lane.  Classes past the last whole chunk come with the last
+    // four.
+    typedef uint32_t u2v __attribute__((ext_vector_type(2), aligned(2)));
     const uint32_t local = tid / 4u, g = tid % 4u, a = run * kRun + local, nch = p.nc / 4u;
     uint32_t kb = kPad, ks = kPad, kt = kPad;
     u2v bx = (u2v)0u;
     if (a < p.A) {
       // one image spans fewer than 2^31 elements (checked on the host)
-      const u2v* row = reinterpret_cast<const u2v*>(img + a * (uint32_t)p.L.sa);
-      if (g == 0) bx = row[0];
+      const uint16_t* row = img + a * (uint32_t)p.L.sa;
+      u2v end = (u2v)0u;
+      if (g == 0) {
+        bx = *reinterpret_cast<const u2v*>(row);
+        if (p.nc % 4u) end = *reinterpret_cast<const u2v*>(row + p.nc);
+      }
       for (uint32_t j0 = g; j0 < nch; j0 += 4u * kRUnroll) {
         u2v v[kRUnroll];
 #pragma unroll
         for (uint32_t u = 0; u < kRUnroll; ++u) {
           const uint32_t j = j0 + 4u * u;
-          v[u] = j < nch ? row[1u + j] : (u2v)0u;
+          v[u] = j < nch ? *reinterpret_cast<const u2v*>(row + 4u + 4u * j) : (u2v)0u;
         }
 #pragma unroll
         for (uint32_t u = 0; u < kRUnroll; ++u) {
@@ -1701,6 +1707,14 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
               fold3(kb, ks, kt, (kw & 0xffff0000u) | (c + 1u));
             }
           }
+        }
+      }
+      if (p.nc % 4u && g == 0) {  // classes nc - 4 + e
+#pragma unroll
+        for (uint32_t q = 0; q < 2; ++q) {
+          const uint32_t w = end[q], kw = run_key2(w), c = p.nc - 4u + 2u * q;
+          if (c >= 4u * nch) fold3(kb, ks, kt, (kw << 16) | c);
+          if (c + 1u >= 4u * nch) fold3(kb, ks, kt, (kw & 0xffff0000u) | (c + 1u));
         }
       }
     }
@@ -2164,9 +2178,10 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
 
   // Fallback: every stage-1 row into the LDS table (thread (grow, cls): class
   // cls of ranks grow, grow + G, ...); pairs keyed at most T1 survive.
-  if (tid == 0) count = 0;
+  if (tid == 0) count = count2 = 0;
   __syncthreads();
   if (grow < G) {
+    uint32_t at_t1 = 0;
     for (uint32_t r0 = grow; r0 < K; r0 += G * kGatherBatch) {
       uint32_t h[kGatherBatch];
 #pragma unroll
@@ -2185,10 +2200,12 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
           if (key <= T1) {
             const uint32_t slot = atomicAdd(&count, 1u);
             if (slot < kSortCap) s2buf[slot] = (key << 16) | f;
+            at_t1 += key == T1;
           }
         }
       }
     }
+    if (at_t1) atomicAdd(&count2, at_t1);
   }
   __syncthreads();
   // the survivors sorted, or (more than kSortCap: ties) K of them: the pairs
@@ -2199,15 +2216,10 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   if (S <= kSortCap) {
     have2 = S;
   } else {
-    const uint32_t pairs = K * nc, lane = tid & 63u, wave = tid >> 6;
-    __syncthreads();  // S is read
-    if (tid == 0) count = count2 = 0;
+    const uint32_t pairs = K * nc, L = S - count2, lane = tid & 63u, wave = tid >> 6;
     __syncthreads();
-    uint32_t less = 0;
-    for (uint32_t i = tid; i < pairs; i += kFinishThreads) less += run_key(table[i]) < T1;
-    if (less) atomicAdd(&count, less);
+    if (tid == 0) count2 = 0;
     __syncthreads();
-    const uint32_t L = count;
     // the pairs at most `top` into the slots from 0 on (at most K of them)
     auto take = [&](uint32_t top) {
       for (uint32_t i = tid; i < pairs; i += kFinishThreads) {
@@ -2514,11 +2526,7 @@ thin_status select_run(const thin_desc* decoded, int64_t max_det, bool agn, void
     rp.rows_per = w.two.rows_per;
     rp.agnostic = agn ? 1 : 0;
     rp.vec_classes = vec_classes ? 1 : 0;
-    rp.row_classes = !vec_classes && decoded->strides[2] == 1 && decoded->strides[1] % 4 == 0 && nc % 4 == 0 &&
-                             (B == 1 || decoded->strides[0] % 4 == 0) &&
-                             reinterpret_cast<uintptr_t>(decoded->data) % 8 == 0
-                         ? 1
-                         : 0;
+    rp.row_classes = !vec_classes && decoded->strides[2] == 1 && nc >= 4 ? 1 : 0;
     rp.runs_rec = reinterpret_cast<uint32_t*>(ws + w.runs);
     rp.runs_side = reinterpret_cast<uint16_t*>(ws + w.runs_side);
     rp.info = reinterpret_cast<u4v*>(ws + w.info);
