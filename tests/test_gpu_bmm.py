@@ -243,18 +243,18 @@ def _operand(form, batch, rows, k, g, device):
     return t[:, :, ::2], t.to(device)[:, :, ::2]
 
 
-@pytest.mark.parametrize("batch,m,n", [(2, 33, 31), (1, 47, 100), (130, 66, 70), (1, 1472, 1470)])
-@pytest.mark.parametrize("k", [1, 31, 32, 34, 64, 67, 130, 259])
+@pytest.mark.parametrize("batch,m,n,k", [(*shape, k) for shape in ((2, 33, 31), (1, 47, 100), (130, 66, 70), (1, 1472, 1470))
+                                         for k in (1, 31, 32, 34, 64, 67, 130, 259)
+                                         if shape[0] * shape[1] * shape[2] * k <= 130 * 66 * 70 * 130])
 @pytest.mark.parametrize("fa,fb", [("steps", "steps"), ("rows", "rows"), ("steps", "rows"), ("rows", "steps"),
                                    ("neither", "rows"), ("steps", "neither")])
 def test_bmm_load_forms(gpu, batch, m, n, k, fa, fb):
     """Every pair of operand load forms at both tile sizes (the last two shapes
     give 512 or more 64 x 64 tiles), with partial row tiles, reductions around
     the 32, 64 and 128-step chunks and remainders of 4 and 8 steps, operands at
-    2-byte alignment: the bits of the sequential sum."""
+    2-byte alignment: the bits of the sequential sum.  (The largest shapes only
+    as far as the oracle is quick.)"""
     from thintnpu_amd import capi
-    if batch * m * n * k > 130 * 66 * 70 * 130:
-        pytest.skip("the same chunk counts run at the smaller shapes")
     g = gen(batch * 7 + m + k)
     a, ad = _operand(fa, batch, m, k, g, gpu)
     b, bd = _operand(fb, batch, n, k, g, gpu)
@@ -284,31 +284,30 @@ def _blocked(batch, channels, tokens, c0, g):
 
 
 @pytest.mark.parametrize("c0", [8, 16, 32])
-@pytest.mark.parametrize("count", [9, 12, 17, 20, 23, 33, 36, 39, 131])
-def test_blocked_step_tails(gpu, c0, count):
+@pytest.mark.parametrize("origin", [0, 8])
+def test_blocked_step_tails(gpu, c0, origin):
     """Reductions over blocked channels whose count is no multiple of 8: the
     steps after the last whole run of 8 lie in their own block, not behind the
-    run before them.  From origin 0 and 8, with q^T k, one blocked and one
-    plain operand either way round, heads of one tensor, and 512 or more
-    64 x 64 tiles."""
+    run before them.  q^T k, one blocked and one plain operand either way
+    round, heads of one tensor, and 512 or more 64 x 64 tiles."""
     from thintnpu_amd import capi
-    g = gen(c0 * 1000 + count)
-    for origin in (0, 8):
+    for count in (9, 12, 17, 20, 23, 33, 36, 39, 131):
+        g = gen(c0 * 1000 + count)
         for batch, tokens in ((2, 41), (130, 70)):
             x, y = _blocked(batch, origin + count, tokens, c0, g), _blocked(batch, origin + count, tokens, c0, g)
             xd, yd = x.to(gpu), y.to(gpu)
             args = (True, False, False, 0, origin, count, origin, count)
-            assert bits_equal(capi.layout_bmm(xd, yd, *args), ob.layout_bmm(x, y, *args))
+            assert bits_equal(capi.layout_bmm(xd, yd, *args), ob.layout_bmm(x, y, *args)), count
         plain = torch.randn(130, 37, count, generator=g).half()
         args = (False, False, False, 0, 0, -1, origin, count)
-        assert bits_equal(capi.layout_bmm(plain.to(gpu), yd, *args), ob.layout_bmm(plain, y, *args))
+        assert bits_equal(capi.layout_bmm(plain.to(gpu), yd, *args), ob.layout_bmm(plain, y, *args)), count
         right = plain.transpose(1, 2)
         args = (True, False, False, 0, origin, count)
-        assert bits_equal(capi.layout_bmm(xd, plain.to(gpu).transpose(1, 2), *args), ob.layout_bmm(x, right, *args))
+        assert bits_equal(capi.layout_bmm(xd, plain.to(gpu).transpose(1, 2), *args), ob.layout_bmm(x, right, *args)), count
         group = (origin + count + 31) // 32 * 32
         heads = _blocked(1, 3 * group, 50, c0, g)
         args = (True, False, False, 3, origin, count, origin, count)
-        assert bits_equal(capi.layout_bmm(heads.to(gpu), heads.to(gpu), *args), ob.layout_bmm(heads, heads, *args))
+        assert bits_equal(capi.layout_bmm(heads.to(gpu), heads.to(gpu), *args), ob.layout_bmm(heads, heads, *args)), count
 
 
 @pytest.mark.parametrize("c0", [8, 24, 40, 64, 128])
@@ -346,24 +345,53 @@ def test_partial_rows(gpu, batch, rows, k):
 
 
 @pytest.mark.parametrize("batch,m,n", [(3, 1, 5), (2, 40, 70), (700, 8, 65), (650, 16, 33), (650, 17, 33), (2100, 5, 70)])
-@pytest.mark.parametrize("k", [1, 8, 21, 32, 33, 40, 64, 77, 136, 520, 528])
-def test_columns_in_vectors(gpu, batch, m, n, k):
+def test_columns_in_vectors(gpu, batch, m, n):
     """Columns of b in aligned vectors along k, at sizes on both sides of the
     choice between chains of fmas and matrix tiles: one to four rows a wave,
     reductions around the staging rounds, rows of a adjacent (gathered below
     8, which leaves the tiled chains) or not, columns a line apart or not."""
     from thintnpu_amd import capi
-    if batch * m * n * k > 700 * 16 * 65 * 136:
-        batch = 2
-    g = gen(batch + m + n + k)
-    pitch = (k + 7) // 8 * 8
-    store = torch.randn(batch, n, pitch, generator=g).half()
-    b, bd = store[:, :, :k].transpose(1, 2), store.to(gpu)[:, :, :k].transpose(1, 2)
-    a = torch.randn(batch, m, k, generator=g).half()
+    for k in (1, 8, 21, 32, 33, 40, 64, 77, 136, 520, 528):
+        entries = batch if batch * m * n * k <= 700 * 16 * 65 * 136 else 2
+        g = gen(batch + m + n + k)
+        store = torch.randn(entries, n, (k + 7) // 8 * 8, generator=g).half()
+        b, bd = store[:, :, :k].transpose(1, 2), store.to(gpu)[:, :, :k].transpose(1, 2)
+        a = torch.randn(entries, m, k, generator=g).half()
+        expect = ob.sequential_bmm(a, b)
+        assert bits_equal(capi.bmm(a.to(gpu), bd), expect), k
+        rows = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+        assert bits_equal(capi.bmm(rows, bd), expect), k
+
+
+@pytest.mark.parametrize("batch,m,n", [(2, 40, 70), (130, 66, 70)])
+@pytest.mark.parametrize("k", [20, 40, 67, 140])
+def test_specials_in_matrix_tiles(gpu, batch, m, n, k):
+    """Infinities, NaN, signed zeros, subnormals and the largest values among
+    ordinary ones, in both tile sizes of the short and the long reduction, with
+    operands loaded along steps and along rows."""
+    from thintnpu_amd import capi
+    vals = torch.tensor([0., -0., float("inf"), -float("inf"), float("nan"), 2 ** -24, -2 ** -24, 3 * 2 ** -20, 65504.,
+                         -65504.]).half()
+    g = gen(batch + k)
+
+    def operand(*shape):
+        x = torch.randn(shape, generator=g).half()
+        special = vals[torch.randint(0, len(vals), shape, generator=g)]
+        return torch.where(torch.rand(shape, generator=g) < 0.5 / k, special, x)
+
+    a, b = operand(batch, m, k), operand(batch, k, n)
     expect = ob.sequential_bmm(a, b)
-    assert bits_equal(capi.bmm(a.to(gpu), bd), expect)
-    rows = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
-    assert bits_equal(capi.bmm(rows, bd), expect)
+    assert expect.isnan().any() and expect.isinf().any() and expect.isfinite().any()
+    for ta in (False, True):
+        ad = a.transpose(1, 2).contiguous().to(gpu).transpose(1, 2) if ta else a.to(gpu)
+        for tb in (False, True):
+            bd = b.transpose(1, 2).contiguous().to(gpu).transpose(1, 2) if tb else b.to(gpu)
+            assert same_bits(capi.bmm(ad, bd), expect), (ta, tb)
+    # sums that stay subnormal, and -0 from negative underflow
+    a, b = (torch.randn(batch, m, k, generator=g) * 2 ** -12).half(), (torch.randn(batch, k, n, generator=g) * 2 ** -11).half()
+    expect = ob.sequential_bmm(a, b)
+    assert (expect.view(torch.int16) == -32768).any()
+    assert bits_equal(capi.bmm(a.to(gpu), b.to(gpu)), expect)
 
 
 @pytest.mark.parametrize("entries,m,k,pitch,step", [(24, 17, 8, 8, 1), (24, 17, 72, 72, 1), (24, 1, 40, 72, 1),

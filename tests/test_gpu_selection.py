@@ -135,6 +135,18 @@ def test_selection_every_encoding_two_launch(gpu, layout, agnostic, max_det):
     run_case(gpu, x, max_det, agnostic, layout, f"every-encoding-{layout}-{agnostic}-{max_det}")
 
 
+@pytest.mark.parametrize("agnostic", [False, True])
+def test_selection_every_encoding_many_runs(gpu, agnostic):
+    """The same images four times over, in other orders: 512 runs, whose octets
+    128 threads read, with waves of plain scores only and of any."""
+    g = torch.Generator().manual_seed(512)
+    bits = torch.stack([torch.randperm(65536, generator=g) for _ in range(4)]).to(torch.int32).to(torch.int16)
+    bits[3] = bits[3].sort().values  # non-negative encodings apart from the others
+    scores = bits.view(torch.float16).reshape(4, 16384, 4)
+    x = torch.cat((torch.randn(4, 16384, 4, generator=g).half(), scores), -1)
+    run_case(gpu, x, 300, agnostic, "transposed", f"every-encoding-many-{agnostic}")
+
+
 @pytest.mark.parametrize("batch,anchors,nc,max_det", [(2, 129, 4, 100), (2, 257, 12, 300), (3, 1000, 100, 300),
                                                       (1, 3360, 256, 300), (2, 8400, 80, 300), (1, 1, 4, 300),
                                                       (3, 7, 8, 5), (1, 500, 1024, 32)])
@@ -147,6 +159,23 @@ def test_selection_row_form(gpu, batch, anchors, nc, max_det, agnostic):
     from tests.selection_fixtures import predictions
     x = predictions(batch, anchors, nc, seed=anchors + nc)
     run_case(gpu, x, max_det, agnostic, "contiguous", f"row-{batch}x{anchors}x{nc}-{agnostic}")
+
+
+@pytest.mark.parametrize("batch,anchors,nc,max_det", [(2, 129, 4, 100), (2, 257, 5, 300), (1, 1000, 30, 300),
+                                                      (1, 500, 99, 200), (1, 20000, 7, 300), (1, 300, 1023, 30)])
+@pytest.mark.parametrize("agnostic", [False, True])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+def test_selection_row_form_tails(gpu, batch, anchors, nc, max_det, agnostic, offset):
+    """Rows of any class count from 4 on, at odd offsets and pitches."""
+    from tests.selection_fixtures import predictions
+    from thintnpu_amd import capi
+    x = predictions(batch, anchors, nc, seed=anchors + nc)
+    wide = torch.zeros(batch, anchors, nc + 9, dtype=torch.float16)
+    wide[:, :, offset:offset + 4 + nc] = x
+    out, tr = capi.detection_select(wide.to(gpu)[:, :, offset:offset + 4 + nc], max_det, agnostic, trace=["class_max", "stage1"])
+    ref = sel.select(x, max_det, agnostic)
+    assert bits_equal(out.cpu(), ref["output"])
+    assert bits_equal(tr["class_max"].cpu(), ref["class_max"]) and torch.equal(tr["stage1"].cpu(), ref["stage1_indices"])
 
 
 @pytest.mark.parametrize("noalloc", [False, True])
