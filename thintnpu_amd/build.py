@@ -38,12 +38,12 @@ HIP_FLAGS = [
     # the kernels spell out (e.g. the unfused-chain intermediates) survives.
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # matrix accumulators in VGPRs: no copies between the register halves around
-    # short product loops
-    "-mllvm", "-amdgpu-mfma-vgpr-form",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
     f"-I{INCLUDE}", f"-I{HIP_SRC}",
 ]
+# Flags of single sources.  bmm: matrix accumulators in VGPRs, no copies between
+# the register halves around short product loops.
+SOURCE_FLAGS = {"bmm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:
@@ -68,7 +68,7 @@ def build_hip(verbose: bool = False) -> Path:
 
     def compile_one(src: Path) -> Path:
         obj = obj_dir / (src.name + ".o")
-        cmd = [HIPCC, *HIP_FLAGS, "-x", "hip", "-c", str(src), "-o", str(obj)]
+        cmd = [HIPCC, *HIP_FLAGS, *SOURCE_FLAGS.get(src.name, []), "-x", "hip", "-c", str(src), "-o", str(obj)]
         if verbose:
             print(" ".join(cmd), file=sys.stderr)
         _run(cmd)
