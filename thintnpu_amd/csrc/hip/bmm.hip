@@ -224,7 +224,7 @@ struct Stage {
 
   __device__ __forceinline__ void store(const Side& s, float* lds, Regs& v) const {
     if constexpr (RF) {
-      if (s.ragged && across() == s.rows / 8u) {
+      if (__builtin_expect(s.ragged != 0u, 0) && across() == s.rows / 8u) {
 #pragma unroll
         for (uint32_t u = 0; u < kPer; ++u) v[u] = tail_first(v[u], s.ragged);
       }
@@ -382,12 +382,13 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
   const char* bq = SQ::base(p.Q, bt);
   sp.aim(p.P, bt, p0, 0, K);
   sq.aim(p.Q, bt, q0, 0, K);
-  uint32_t n = 0;  // the next chunk to load
+  uint32_t n = 0;                             // the next chunk to load
+  const uint32_t anew = p.walk ? 0u : last;  // chunks from this to the last take their offsets anew
   // chunk n into register set n % PF; past the last chunk that one again,
   // which nothing stores: a test around the loads would leave the waits
   // without a count of the loads behind the one they wait for
   auto load = [&](int set) __attribute__((always_inline)) {
-    if (n == last || (p.walk && n < last)) {
+    if (n - anew <= last - anew) {
       sp.aim(p.P, bt, p0, n * KD, K);
       sq.aim(p.Q, bt, q0, n * KD, K);
       bp = SP::base(p.P, bt);
