@@ -222,9 +222,10 @@ struct Stage {
     }
   }
 
+  template <bool ODD>
   __device__ __forceinline__ void store(const Side& s, float* lds, Regs& v) const {
-    if constexpr (RF) {
-      if (__builtin_expect(s.ragged != 0u, 0) && across() == s.rows / 8u) {
+    if constexpr (RF && ODD) {
+      if (s.ragged && across() == s.rows / 8u) {
 #pragma unroll
         for (uint32_t u = 0; u < kPer; ++u) v[u] = tail_first(v[u], s.ragged);
       }
@@ -357,7 +358,11 @@ struct Const {
 // matrix pipe is busy 55-60% of the launch, at [128,64,400] x [128,400,400]
 // 36.4 us (72 TFLOP/s; 80.5 us with the fma chains this replaced) against the
 // 17 us that the products alone take at 153 TFLOP/s.
-template <int KD, int W, bool PR, bool QR>
+//
+// ODD: blocks that do not divide a chunk, or rows of one tile that end in a
+// partial run (walk, ragged).  With their tests in every product's loop, v p^T
+// of 1600 tokens took 20.7-21.8 us instead of 20.4.
+template <int KD, int W, bool PR, bool QR, bool ODD>
 __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPlan p) {
   constexpr int R = 32 * W;
   using SP = Stage<PR, KD, R, W>;
@@ -382,15 +387,14 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
   const char* bq = SQ::base(p.Q, bt);
   sp.aim(p.P, bt, p0, 0, K);
   sq.aim(p.Q, bt, q0, 0, K);
-  uint32_t n = 0;                             // the next chunk to load
-  const uint32_t anew = p.walk ? 0u : last;  // chunks from this to the last take their offsets anew
+  uint32_t n = 0;  // the next chunk to load
   // chunk n into register set n % PF; past the last chunk that one again,
   // which nothing stores: a test around the loads would leave the waits
   // without a count of the loads behind the one they wait for
   auto load = [&](int set) __attribute__((always_inline)) {
-    if (n - anew <= last - anew) {
-      sp.aim(p.P, bt, p0, n * KD, K);
-      sq.aim(p.Q, bt, q0, n * KD, K);
+    if (n == last || (ODD && n < last && p.walk)) {
+      sp.aim(p.P, bt, p0, ODD ? n * KD : last * KD, K);
+      sq.aim(p.Q, bt, q0, ODD ? n * KD : last * KD, K);
       bp = SP::base(p.P, bt);
       bq = SQ::base(p.Q, bt);
     }
@@ -426,8 +430,8 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
       sp.trim(p.P, last * KD, K, vp[set]);
       sq.trim(p.Q, last * KD, K, vq[set]);
     }
-    sp.store(p.P, to, vp[set]);
-    sq.store(p.Q, to + SP::kFloats, vq[set]);
+    sp.template store<ODD>(p.P, to, vp[set]);
+    sq.template store<ODD>(p.Q, to + SP::kFloats, vq[set]);
   };
   // chunk c = S mod PF from its buffer, chunk c + 1 into the other
   auto step = [&](auto S) __attribute__((always_inline)) {
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
 // and stores of this one.  At [128,400,32] x [128,32,400] 23.8 us (96.9 with
 // the fma chains this replaced): 9 us of it without products and stores, the
 // products add 11 and the stores of 41 MB 3.
-template <int W, bool PR, bool QR>
+template <int W, bool PR, bool QR, bool ODD>
 __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   constexpr int KD = 32, R = 32 * W;
   using SP = Stage<PR, KD, R, W>;
@@ -522,8 +526,8 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     sq.trim(p.Q, 0, K, vq);
     sp.trim(p.P, 0, K, vp);
   }
-  sq.store(p.Q, lds, vq);
-  sp.store(p.P, ldsp, vp);
+  sq.template store<ODD>(p.Q, lds, vq);
+  sp.template store<ODD>(p.P, ldsp, vp);
   __syncthreads();
   typename OQ::Group gq;
   oq.read(gq, lds, 0);
@@ -545,7 +549,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     const uint32_t pr = p0 + wp;
     if (more) {
       p0 = tile_row<PR>(p.P, pt + 1u, p.ptiles, R);
-      if (pt + 2u == p.ptiles || p.walk) {
+      if (pt + 2u == p.ptiles || (ODD && p.walk)) {
         sp.aim(p.P, bt, p0, 0, K);
         bp = SP::base(p.P, bt);
       } else {
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
     // [128,400,32] x [128,32,400])
     if (more) {
       if (K < KD) sp.trim(p.P, 0, K, vp);
-      sp.store(p.P, ldsp + kTo, vp);
+      sp.template store<ODD>(p.P, ldsp + kTo, vp);
     }
     if (work) {
       if (p.y_vec && pt + 1u < p.ptiles) {
@@ -668,10 +672,15 @@ __global__ __launch_bounds__(kBmmThreads) void bmm_gather_kernel(BmmPlan p) {
 
 template <bool SHORT, int W, bool PR, bool QR>
 void launch_form(const BmmPlan& p, uint32_t grid, hipStream_t stream) {
-  if constexpr (SHORT)
-    hipLaunchKernelGGL((bmm_short_kernel<W, PR, QR>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
-  else
-    hipLaunchKernelGGL((bmm_kernel<bmm_depth(W), W, PR, QR>), dim3(grid), dim3(kBmmThreads), 0, stream, p);
+  const bool odd = p.walk || p.P.ragged || p.Q.ragged;
+  const dim3 g(grid), t(kBmmThreads);
+  if constexpr (SHORT) {
+    if (odd) hipLaunchKernelGGL((bmm_short_kernel<W, PR, QR, true>), g, t, 0, stream, p);
+    else hipLaunchKernelGGL((bmm_short_kernel<W, PR, QR, false>), g, t, 0, stream, p);
+  } else {
+    if (odd) hipLaunchKernelGGL((bmm_kernel<bmm_depth(W), W, PR, QR, true>), g, t, 0, stream, p);
+    else hipLaunchKernelGGL((bmm_kernel<bmm_depth(W), W, PR, QR, false>), g, t, 0, stream, p);
+  }
 }
 
 template <bool SHORT, int W>
@@ -1302,7 +1311,7 @@ extern "C" thin_status thin_layout_bmm(const thin_desc* a, const thin_desc* b, c
     x->last_rows = x->row.blk.d == 1 ? x->rows - 8u : (x->rows - 1u) & ~7u;
     const uint32_t part = x->row.blk.d == 1 ? x->rows & 7u : 0u;
     if (x->rows > r) x->early = part ? 8u - part : 0u;
-    else x->ragged = part;
+    else x->ragged = x == &p.P ? (pr ? part : 0u) : (qr ? part : 0u);
   }
   p.P.steps_near = unit_step(p.P.step) <= unit_step(p.P.row);
   p.Q.steps_near = unit_step(p.Q.step) <= unit_step(p.Q.row);
