@@ -275,8 +275,10 @@ thin_status thin_detection_select(const thin_desc* decoded, int64_t max_det, int
  * and errors as thin_detection_select; the intermediates live in a static
  * device array of the library, one per GPU, whose device address is taken
  * once per device on the first call with that device current.  Calls whose
- * thin_detection_select_workspace(...) exceeds THIN_SELECT_SCRATCH_BYTES fail
- * with THIN_ERR_WORKSPACE.  Allocates nothing (no hipMalloc, hipFree or
+ * intermediates do not fit THIN_SELECT_SCRATCH_BYTES fail with
+ * THIN_ERR_WORKSPACE; sizes whose thin_detection_select_workspace(...) exceeds
+ * it but which a path of several launches serves with less take that path.
+ * Allocates nothing (no hipMalloc, hipFree or
  * allocating library call).  Every call on one GPU shares that GPU's scratch:
  * calls that overlap on one GPU (two streams, or two host threads) race and
  * must be ordered by the caller. */

@@ -354,10 +354,12 @@ struct Const {
 // the products of this one (one: 41.2 against 36.4 us for the batched v p^T,
 // four: 40.7).
 //
-// Bound by the issue of the products and of the VALU work beside them: the
-// matrix pipe is busy 55-60% of the launch, at [128,64,400] x [128,400,400]
-// 36.4 us (72 TFLOP/s; 80.5 us with the fma chains this replaced) against the
-// 17 us that the products alone take at 153 TFLOP/s.
+// Bound by the issue of the products and of the VALU work beside them: at
+// [128,64,400] x [128,400,400] the matrix pipe is busy 41,600 of the 77,700
+// cycles that the launch keeps a shader engine busy (54%).  34.3 us back to back
+// on the same operands, 37.8 in a kernel trace over changing ones (80.5 with the
+// fma chains this replaced), against the 17 us that the products alone take at
+// 153 TFLOP/s.
 //
 // ODD: blocks that do not divide a chunk, or rows of one tile that end in a
 // partial run (walk, ragged).  With their tests in every product's loop, v p^T
@@ -485,9 +487,9 @@ __global__ __launch_bounds__(kBmmThreads, W == 2 ? 3 : 2) void bmm_kernel(BmmPla
 
 // The same for K <= 32 (one chunk): the block keeps its Q operand in registers
 // and walks `span` P tiles, the next tile's loads in flight under the products
-// and stores of this one.  At [128,400,32] x [128,32,400] 23.8 us (96.9 with
+// and stores of this one.  At [128,400,32] x [128,32,400] 24.4 us (96.9 with
 // the fma chains this replaced): 9 us of it without products and stores, the
-// products add 11 and the stores of 41 MB 3.
+// products add 11 and the stores of 41 MB 3 to 4.
 template <int W, bool PR, bool QR, bool ODD>
 __global__ __launch_bounds__(kBmmThreads) void bmm_short_kernel(BmmPlan p) {
   constexpr int KD = 32, R = 32 * W;

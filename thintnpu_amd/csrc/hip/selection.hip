@@ -1241,15 +1241,16 @@ __global__ __launch_bounds__(kSplitThreads) void merge2_kernel(SplitPlan p) {
 // ---------------------------------------------------------------- two-launch selection
 // The selection in two launches, for images of up to kMaxRuns * kRun anchors:
 //
-//   runs   (grid runs x B, 512 threads): per anchor of kRun, the three
-//          smallest (key << 16 | class) over the classes; the run's
+//   runs   (grid runs x B, 512 threads; 128 where there are many runs): per
+//          anchor of kRun, the three smallest (key << 16 | class) over the
+//          classes; the run's
 //          (key << 16 | anchor) records sorted (a bitonic network over two
 //          waves) -> runs_rec, with each record's row key (below) ->
 //          runs_side; per anchor a 16-byte info record (box, class-max score
 //          bits and class, second key and class) -> info.
 //   finish (grid B, 1024 threads): the stage-1 candidates of the sorted runs
-//          (a bound by the rank of their q-th records), sorted, while the info of
-//          every candidate and the score rows of the few candidates whose
+//          (a bound by the rank of their q-th records), sorted, while the info
+//          of every candidate and the score rows of the few candidates whose
 //          third key could reach the bound are in flight; stage 2 from the K
 //          class-max pairs, the second pairs and those rows; rows packed
 //          from LDS.
@@ -1262,19 +1263,21 @@ __global__ __launch_bounds__(kSplitThreads) void merge2_kernel(SplitPlan p) {
 // ones.  A second pair's score bits follow from its key, except for NaN and
 // zero keys (several encodings each): rows with such a second key are
 // prefetched too.  A run record's row key is the smallest key that makes its
-// row needed: the third key, or the second key when that is NaN or zero.  When the rows do not fit (thousands of tied scores), or a
-// trace of the gathered scores is asked for, every stage-1 row is gathered
-// into an LDS table instead, and ties beyond kSortCap survivors go through a
-// radix select of the K-th smallest pair.
+// row needed: the third key, or the second key when that is NaN or zero.  When
+// the rows do not fit (thousands of tied scores), or a trace of the gathered
+// scores is asked for, every stage-1 row is gathered into an LDS table instead.
+// Of more than kSortCap survivors, those below T1 and the first ties at T1 in
+// pair order are taken, or, where the former are more than K, the records up to
+// the K-th smallest, found by a radix select.
 //
 // Sorting in one workgroup is a bitonic network over at most kSortCap
 // records, held by four waves (E records per thread for n = 256E; smaller n a
 // record per thread): exchanges within a thread in registers, within a wave
 // by DPP and permlane swaps, between waves through LDS.  More stage-1
-// candidates than kSortCap go through an exact radix select of the K-th
-// smallest record first (four 8-bit digits, LDS histograms), so only K
-// records are sorted.  Records are unique, so the network's order is the
-// stable (key, index) order.
+// candidates than kSortCap (after a second bound, see finish_kernel) go through
+// an exact radix select of the K-th smallest record first (four 8-bit digits,
+// LDS histograms), so only K records are sorted.  Records are unique, so the
+// network's order is the stable (key, index) order.
 constexpr uint32_t kRun = 128;             // anchors per sorted run
 constexpr uint32_t kRunThreads = 512;      // runs_kernel workgroups of a few images
 constexpr uint32_t kRunManyThreads = 128;  // and of many runs
@@ -1288,9 +1291,9 @@ constexpr uint32_t kMaxX = 256;            // prefetched candidate rows
 constexpr uint32_t kXTable = 16384;        // their fp16 scores in LDS
 constexpr uint32_t kXBatch = 8;            // prefetched row loads per thread
 constexpr uint32_t kNoX = 0xffffu;
-// finish_kernel's reused LDS region (32-bit words): the candidate tables,
-// then (fallback) the pair table; info1 lies past the pair table and survives
-// it.
+// finish_kernel's reused LDS region (32-bit words): the tables of candidate
+// slots, whose place (fallback) the pair table takes; info1 lies past the pair
+// table and survives it.
 constexpr uint32_t kRegInfoSlot = 8192;                        // u4v [kSortCap]: info per slot
 constexpr uint32_t kRegXTable = kRegInfoSlot + 4 * kSortCap;   // u16 [kXTable]
 constexpr uint32_t kRegInfo1 = kRegXTable + kXTable / 2;       // u4v [kSplitMaxK]: info per stage-1 rank
@@ -1587,9 +1590,10 @@ __device__ __forceinline__ void fold_word(uint32_t w, uint32_t c, uint32_t& b0, 
 // run's records sorted: waves 0 and 1 sort 64 each (ascending, descending),
 // one LDS exchange at distance 64 and the in-wave end of the last merge.
 //
-// kRunManyThreads: the octet form alone, eight class groups in 15 KB of LDS
-// instead of 32 in 66 KB, for launches of many runs: ten groups of waves fit a
-// compute unit where two did, and a run merges a quarter of the triples.
+// kRunManyThreads: the octet form alone, eight class groups in 14 KB of LDS
+// instead of 32 in 56 KB, for launches of many runs: ten runs at a time fit a
+// compute unit (5 waves a SIMD by their 96 registers) instead of two, and a run
+// merges a quarter of the triples.
 template <uint32_t kRunThreads>
 __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
   constexpr bool kMany = kRunThreads == kRunManyThreads;
@@ -1848,6 +1852,13 @@ __global__ __launch_bounds__(kRunThreads) void runs_kernel(RunsPlan p) {
 // kernel did, left 760 candidates of 8400 anchors for K = 300 on average and
 // over 1024 for one image in thirty, which then took the radix select and
 // the full gather: 44 us for a batch of 32 images, 10 for one image.
+//
+// One image of 8400 anchors x 80 classes, K = 300 (363 candidates, no rows to
+// prefetch), 8.4 us: records loaded 0.84, ranks 0.68, counts 0.68, scan 0.24,
+// candidates written and their info requested 1.56, sort of 512 1.36, stage-1
+// ranks 0.92, extras 0.16, merge and rows 1.92.  Each phase is a latency with a
+// barrier behind it.  4 images of 33600 anchors: 13.4 us, the ranks of 263 runs
+// 3.9 of them.
 template <bool WIDE>
 __global__ __launch_bounds__(kFinishThreads) void finish_kernel(RunsPlan p) {
   __shared__ __attribute__((aligned(16))) uint32_t region[kRegWords];
