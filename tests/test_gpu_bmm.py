@@ -414,3 +414,34 @@ def test_more_products_than_a_launch(gpu, entries, m, k, pitch, step):
     capi.bmm(a, b.expand(batch, 1, k).transpose(1, 2), out=out)
     expect = acc.half().view(torch.int16).unfold(0, m, 1)
     assert torch.equal(out[:, :, 0].view(torch.int16), expect)
+
+
+@pytest.mark.parametrize("heads,tokens", [(8, 24), (4, 16), (300, 72)])
+def test_blocked_output_of_few_channels(gpu, heads, tokens):
+    """v p^T of 16 channels a head into the blocked layout, heads of one tensor
+    and one tensor a head, at sizes that take the chains of fmas."""
+    from thintnpu_amd import capi
+    g = gen(heads + tokens)
+    p = torch.randn(heads, tokens, tokens, generator=g).half()
+    x = torch.randn(1, heads, tokens, 16, generator=g).half()
+    args = (False, True, True, heads, 0, 16)
+    assert bits_equal(capi.layout_bmm(x.to(gpu), p.to(gpu), *args), ob.layout_bmm(x, p, *args))
+    x = x.transpose(0, 1).contiguous()
+    args = (False, True, True)
+    assert bits_equal(capi.layout_bmm(x.to(gpu), p.to(gpu), *args), ob.layout_bmm(x, p, *args))
+
+
+@pytest.mark.parametrize("heads,tokens", [((1 << 24) + 16, 1), ((1 << 26) + 16, 8)])
+def test_more_heads_than_a_launch(gpu, heads, tokens):
+    """The same beyond one launch, a channel a head into blocks of 16 heads:
+    gathered elements, and chains."""
+    from thintnpu_amd import capi
+    g = torch.Generator(device=gpu).manual_seed(7)
+    x = torch.randn(1, heads // 16, tokens, 16, generator=g, device=gpu, dtype=torch.float16)
+    b = torch.randn(heads, 1, tokens, generator=g, device=gpu, dtype=torch.float16)
+    out = torch.full((1, heads // 16, 1, 16), 7.0, device=gpu, dtype=torch.float16)
+    capi.layout_bmm(x, b.transpose(1, 2), False, False, True, heads, 0, 1, out=out)
+    acc = torch.zeros(heads, device=gpu)
+    for t in range(tokens):
+        acc += x[0, :, t].reshape(-1).float() * b[:, 0, t].float()
+    assert torch.equal(out.reshape(-1).view(torch.int16), acc.half().view(torch.int16))
